@@ -407,7 +407,6 @@ struct Ctx final : CtxBase {
     flux.alloc(sizeof(C) * fsz * 2 * nl);
     phys.alloc(sizeof(T) * (size_t)nx * ny * 4 * nl);
     jl.alloc(sizeof(C) * (size_t)nkr * ny * nl);
-    twx.alloc(sizeof(C) * nx); twy.alloc(sizeof(C) * ny);
     upload_twiddles(twx, nx); upload_twiddles(twy, ny);
     build_model();
     build_stepper();
@@ -479,12 +478,17 @@ struct Ctx final : CtxBase {
   }
 
   // ---------------- setup helpers ----------------
+  // exp(-2 pi i j/n), j < n; for an n that is not a power of two dft_even's table (gf_fft.hpp): the
+  // n/2 roots exp(-2 pi i j/(n/2)), then exp(-2 pi i j/n) for j < n/2
   void upload_twiddles(DevBuf& b, int n) {
+    const bool gen = !is_pow2(n);
     std::vector<C> h(n);
     for (int i = 0; i < n; ++i) {
-      const long double a = -2.0L * 3.141592653589793238462643383279502884L * i / n;
+      const int j = gen ? (2 * i < n ? 2 * i : i - n / 2) : i;
+      const long double a = -2.0L * 3.141592653589793238462643383279502884L * j / n;
       h[i].re = (T)std::cos(a); h[i].im = (T)std::sin(a);
     }
+    b.alloc(sizeof(C) * n);
     HIPCHECK(dw::copy(b.p, h.data(), sizeof(C) * n, hipMemcpyHostToDevice));
   }
   double krw(int kr) const { return (double)kr * ((2 * M_PI / d.Lx * d.nx) / d.nx); }
@@ -843,6 +847,8 @@ struct Ctx final : CtxBase {
     c.tw = twy.as<C>();
     a.p = sched[0]; b.p = sched[1]; c.p = sched[2];
     if (tunable()) { a.fsplit = split[0]; b.hsplit = split[1]; c.csplit = split[2]; }
+    // columns that are not a power of two long are short (at most GEN_MAX): one field per workgroup row
+    if (nl == 1 && !is_pow2(d.ny)) a.fsplit = 1;
     if (ab3()) {
       // the RHS history of the aliased band enters later steps: every AB3 step is computed in full
       c.ab3_start = ab3_start >= 0 ? ab3_start : stepno < 3;

@@ -316,37 +316,72 @@ __device__ __forceinline__ void fft_forward(cplx<T> (&v)[C][P], cplx<T>* __restr
   stockham<T, N, P, C, 0, 1, LIGHT>(v, lds, t, tw);
 }
 
-// Direct DFT of a length n < N that is not a power of two, in the data layout of fft_forward:
-// thread t holds x[t + TPT q] (zero where t + TPT q >= n) and receives y[k] = sum_j x[j] w^(jk),
-// w = exp(-2 pi i/n), at k = t + TPT q < n (the other slots come back zero).  roots[j] = w^j,
-// j < n, in LDS.  Each thread forms its P outputs from all n inputs (P n complex products), the
-// index j k mod n advanced by k per term; the inputs are read from lds (broadcast across lanes).
+// Transform of an even length n < N that is not a power of two, in the data layout of fft_forward
+// with P = 4: thread t holds x[t + TPT q] (anything where t + TPT q >= n) and receives
+// y[k] = sum_j x[j] w^(jk), w = exp(-2 pi i/n), at k = t + TPT q < n (the other slots come back zero).
+// With m = n/2, a radix-2 step leaves two sums of length m (even and odd k), and each folds its
+// terms j and m - j: E_j = z_j + z_(m-j) takes the cosine, O_j = z_j - z_(m-j) the sine, which serve
+// the outputs k and m - k at once.  Thread t forms outputs t and m - t of both sums: m/2 steps, each
+// of five LDS reads (four shared by the lanes) and 8 FMAs, where the plain sum of P outputs took
+// P n complex products of two reads each (n = 126: 31 steps against 504), and fewer roundings.
+// lds: 2 N slots; roots (LDS): exp(-2 pi i j/m), then exp(-2 pi i j/n), j < m.
 template <typename T, int N, int P>
-__device__ __forceinline__ void dft_direct(cplx<T> (&v)[1][P], cplx<T>* __restrict__ lds, int t, int n,
-                                           const cplx<T>* __restrict__ roots) {
+__device__ __forceinline__ void dft_even(cplx<T> (&v)[1][P], cplx<T>* __restrict__ lds, int t, int n,
+                                         const cplx<T>* __restrict__ roots) {
+  static_assert(P == 4, "each thread forms the outputs of one k");
   constexpr int TPT = N / P;
-  __syncthreads();   // lds is free: every earlier reader of it is done
+  const int m = n / 2, jm = (m - 1) / 2;            // n < N: jm < TPT and m/2 < TPT
+  cplx<T>* eo = lds + N;                             // E, O of the even sum, E, O of the odd one, per j
 #pragma unroll
-  for (int q = 0; q < P; ++q) {
-    const int j = t + TPT * q;
-    if (j < n) lds[j] = v[0][q];
+  for (int q = 0; q < P; ++q)
+    if (t + TPT * q < n) lds[t + TPT * q] = v[0][q];
+  __syncthreads();
+  if (t < jm) {
+    const int j = t + 1;
+    const cplx<T> x0 = lds[j], x1 = lds[j + m], x2 = lds[m - j], x3 = lds[n - j];
+    const cplx<T> a0 = x0 + x1, a1 = x2 + x3;
+    const cplx<T> b0 = cmul(x0 - x1, roots[m + j]), b1 = cmul(x2 - x3, roots[m + m - j]);
+    eo[4 * t + 0] = a0 + a1;
+    eo[4 * t + 1] = a0 - a1;
+    eo[4 * t + 2] = b0 + b1;
+    eo[4 * t + 3] = b0 - b1;
+  }
+  // the terms that have no partner: j = 0 and, for even m, j = m/2 with the factor (-1)^k
+  cplx<T> z0 = lds[0] + lds[m], z1 = lds[0] - lds[m];
+  if ((m & 1) == 0) {
+    const int h = m / 2;
+    cplx<T> h0 = lds[h] + lds[h + m], h1 = cmul(lds[h] - lds[h + m], roots[m + h]);
+    z0 = (t & 1) ? z0 - h0 : z0 + h0;
+    z1 = (t & 1) ? z1 - h1 : z1 + h1;
+  }
+  __syncthreads();
+  cplx<T> c0 = z0, c1 = z1, d0 = mk((T)0, (T)0), d1 = d0;
+  const bool mine = t <= m / 2;
+  int idx = mine ? t : 0;
+  const int k = idx;
+#pragma unroll 4
+  for (int j = 0; j < jm; ++j) {
+    const cplx<T> w = roots[idx];
+    const cplx<T> E0 = eo[4 * j], O0 = eo[4 * j + 1], E1 = eo[4 * j + 2], O1 = eo[4 * j + 3];
+    c0 = c0 + rmul(w.re, E0);
+    d0 = d0 + rmul(w.im, O0);
+    c1 = c1 + rmul(w.re, E1);
+    d1 = d1 + rmul(w.im, O1);
+    idx += k;
+    if (idx >= m) idx -= m;                          // j k mod m
+  }
+  if (mine) {
+    lds[2 * k] = mk(c0.re - d0.im, c0.im + d0.re);
+    lds[2 * k + 1] = mk(c1.re - d1.im, c1.im + d1.re);
+    if (k > 0 && 2 * k < m) {
+      lds[2 * (m - k)] = mk(c0.re + d0.im, c0.im - d0.re);
+      lds[2 * (m - k) + 1] = mk(c1.re + d1.im, c1.im - d1.re);
+    }
   }
   __syncthreads();
 #pragma unroll
-  for (int q = 0; q < P; ++q) {
-    const int k = t + TPT * q;
-    cplx<T> acc = mk((T)0, (T)0);
-    if (k < n) {
-      int idx = 0;
-      for (int j = 0; j < n; ++j) {
-        acc = acc + cmul(lds[j], roots[idx]);
-        idx += k;
-        if (idx >= n) idx -= n;
-      }
-    }
-    v[0][q] = acc;
-  }
-  __syncthreads();   // lds is free again for the caller
+  for (int q = 0; q < P; ++q) v[0][q] = t + TPT * q < n ? lds[t + TPT * q] : mk((T)0, (T)0);
+  __syncthreads();                                   // lds is free again for the caller
 }
 
 }  // namespace gf

@@ -293,8 +293,8 @@ template <typename T> void launch_from_julia(const Geo<T>& g, const cplx<T>* src
 template <typename T> void launch_mask(const Geo<T>& g, cplx<T>* sol, int nl, hipStream_t s);
 void launch_counter(int64_t* c, int64_t v, int add, hipStream_t s);
 // Grid lengths that are not powers of two (even, 18..GEN_MAX): a column length ny runs in the
-// y-pass kernels of the next power of two with a direct DFT (dft_direct), a row length nx in the
-// x-pass kernel of direct sums (k2_gen_kernel).
+// y-pass kernels of the next power of two, a row length nx in an x-pass kernel of its own
+// (k2_gen_kernel); both transform with dft_even.
 constexpr int GEN_MAX = 256;
 __host__ __device__ constexpr int pow2_ceil(int n) { int m = 1; while (m < n) m *= 2; return m; }
 __host__ __device__ constexpr bool is_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }

@@ -143,12 +143,14 @@ template <int TPT> struct YMap {
 
 // Non-power-of-two column lengths ny (even, up to GEN_MAX) run in separate instantiations
 // (GEN = true) of the y-pass kernels of NY = pow2_ceil(ny): they index with the runtime ny, the
-// rows ny..NY-1 of each thread's points stay unused, and a direct DFT (dft_direct) replaces the
-// Stockham transform, with the ny roots of unity (the global table, which has ny entries) in the
-// LDS twiddle array. The power-of-two kernels keep the constant NY (a runtime ny in them cost
-// 6-7% per step at 64^2-256^2).
+// rows ny..NY-1 of each thread's points stay unused, and dft_even replaces the Stockham transform, in
+// buffers of 2 NY slots (YN), with the ny entries of its global table in the LDS twiddle array.
+// Bound by the latency of its LDS passes: MultiLayerQG 128x126 x 2, per launch, K1 64.9 -> 11.4 us and
+// K3 46.7 -> 12.9 us against the plain sums.  The power-of-two kernels keep the constant NY (a runtime
+// ny in them cost 6-7% per step at 64^2-256^2).
+template <int NY, bool GEN> struct YN { static constexpr int value = GEN ? 2 * NY : NY; };
 template <int NY, int P, bool GEN> struct YTw {
-  static constexpr int size = (GEN && NY > TwPlan<NY, P>::size()) ? NY : TwPlan<NY, P>::size();
+  static constexpr int size = GEN ? NY : TwPlan<NY, P>::size();
 };
 template <typename T, int NY, int P, bool GEN>
 __device__ __forceinline__ void load_y_twiddles(cplx<T>* __restrict__ tw, const cplx<T>* __restrict__ twg, int ny) {
@@ -162,7 +164,7 @@ __device__ __forceinline__ void load_y_twiddles(cplx<T>* __restrict__ tw, const 
 template <typename T, int NY, int P, bool FR, bool GEN>
 __device__ __forceinline__ void y_transform(cplx<T> (&w)[1][P], cplx<T>* __restrict__ L, int t,
                                             const cplx<T>* __restrict__ tw, int ny) {
-  if constexpr (GEN) dft_direct<T, NY, P>(w, L, t, ny, tw);
+  if constexpr (GEN) dft_even<T, NY, P>(w, L, t, ny, tw);
   else fft_forward<T, NY, P, 1, FR>(w, L, t, tw);
 }
 // the column length the y-pass kernels index with
@@ -190,7 +192,7 @@ __device__ __forceinline__ void k1_body(const K1Args<T>& a, int blk, cplx<T>* __
   const bool masked = FS != FS_RAW && !((NL > 1 || MODEL == M_SLQG) && FS == FS_CALCN && a.nomask);
   const bool krk = kr < g.kmax || !masked;
   const T kv = krwave(g, kr);
-  cplx<T>* L = col_buffer<T, NY>(lds, m.slot, m.c);
+  cplx<T>* L = col_buffer<T, YN<NY, GEN>::value>(lds, m.slot, m.c);
   const T nrm = g.inv_norm;
   const int ny = ycol<NY, GEN>(g);
   // masked state value of layer j at y-index l
@@ -299,7 +301,7 @@ __device__ __forceinline__ void k1_body(const K1Args<T>& a, int blk, cplx<T>* __
 template <typename T, int NY, int P, int G, int NL, int MODEL, int FS, bool GEN = false>
 __global__ __launch_bounds__(2 * G * (NY / P)) __attribute__((amdgpu_waves_per_eu(GF_K1_WAVES)))
 void k1_kernel(const K1Args<T> a) {
-  __shared__ cplx<T> lds[G * PairLds<T, NY>::value];
+  __shared__ cplx<T> lds[G * PairLds<T, YN<NY, GEN>::value>::value];
   __shared__ cplx<T> tw[YTw<NY, P, GEN>::size];
   load_y_twiddles<T, NY, P, GEN>(tw, a.tw, a.g.ny);
   __syncthreads();
@@ -646,132 +648,178 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
 }
 
 // ---------------------------------------------------------------------------
-// K2 for rows whose length nx is not a power of two (even, 18..GEN_MAX): one workgroup per row,
-// direct sums over the row's modes and points (O(nx^2) per row) in place of the packed two-row
-// transforms. The same fields, products and outputs as k2_body's modes; the row's half spectra,
-// physical products and the nx roots of unity w^j = exp(-2 pi i j/nx) (the global table) sit in
-// LDS.
+// K2 for rows whose length nx is not a power of two (even, 18..GEN_MAX): the fields, products,
+// packing and outputs of k2_body's modes with the runtime nx in the kernel of NX = pow2_ceil(nx),
+// dft_even in place of the Stockham transform.  Always two rows of one field per transform;
+// a layer (K2_ADVECT_FULL), a product (K2_ADVECT) or a field (forward-in, inverse-out) has its own
+// workgroup row, which these small grids need to fill the GPU.
 // ---------------------------------------------------------------------------
-constexpr int K2G_THREADS = 64;
-template <typename T> struct K2GLds {
-  cplx<T> hs[3][GEN_MAX / 2 + 1];
-  T ph[3][GEN_MAX];
-  cplx<T> roots[GEN_MAX];
+template <int NX> struct K2G {
+  static constexpr int P = 4, TPT = NX / P, G = TPT >= 64 ? 1 : 64 / TPT;
 };
-// c2r of the half spectrum h (columns kr < kin present) at point x: Re h_0 + 2 sum Re(h_k w^-kx)
-// + Re h_(nx/2) (-1)^x; the imaginary parts of the DC and Nyquist columns are ignored, as c2r does
-template <typename T>
-__device__ __forceinline__ T c2r_point(const cplx<T>* h, int kin, int nx, int x, const cplx<T>* roots) {
-  const int kc = kin < nx / 2 + 1 ? kin : nx / 2 + 1;
-  T acc = kc > 0 ? h[0].re : (T)0;
-  int idx = 0;
-  for (int k = 1; k < kc; ++k) {
-    idx += x;
-    if (idx >= nx) idx -= nx;                          // k x mod nx
-    const cplx<T> w = roots[idx];
-    if (2 * k == nx) acc += h[k].re * w.re;
-    else acc += (T)2 * (h[k].re * w.re + h[k].im * w.im);   // 2 Re(h_k conj(w))
-  }
-  return acc;
-}
-// r2c of the physical row p at column kr: sum_x p_x w^(kr x)
-template <typename T>
-__device__ __forceinline__ cplx<T> r2c_point(const T* p, int nx, int kr, const cplx<T>* roots) {
-  cplx<T> acc = czero<T>();
-  int idx = 0;
-  for (int x = 0; x < nx; ++x) {
-    acc = acc + rmul(p[x], roots[idx]);
-    idx += kr;
-    if (idx >= nx) idx -= nx;
-  }
-  return acc;
-}
-template <typename T, int MODE>
-__global__ __launch_bounds__(K2G_THREADS) void k2_gen_kernel(const K2Args<T> a) {
-  __shared__ K2GLds<T> S;
+template <typename T, int NX, int MODE>
+__global__ __launch_bounds__(K2G<NX>::G * K2G<NX>::TPT)
+void k2_gen_kernel(const K2Args<T> a) {
+  constexpr int P = K2G<NX>::P, TPT = K2G<NX>::TPT, G = K2G<NX>::G;
+  constexpr int MAXI = P / 2 + 1;                      // kr = t + i TPT <= nx/2 <= NX/2
+  __shared__ cplx<T> lds[G * 2 * NX];
+  __shared__ cplx<T> tw[NX];
   const Geo<T>& g = a.g;
-  const int nx = g.nx, ny = g.ny, nkr = nx / 2 + 1, t = (int)threadIdx.x, y = (int)blockIdx.x;
-  for (int i = t; i < nx; i += K2G_THREADS) S.roots[i] = a.tw[i];
-  // half spectrum of row y of field f (kr < kin, zero beyond) into S.hs[s]
-  auto load = [&](int s, const cplx<T>* f) {
-    for (int k = t; k < nkr; k += K2G_THREADS) S.hs[s][k] = k < a.kin ? at(f, boff32(k, y, ny)) : czero<T>();
+  const int nx = g.nx, ny = g.ny, t = (int)threadIdx.x % TPT;
+  for (int i = threadIdx.x; i < nx; i += G * TPT) tw[i] = a.tw[i];
+  __syncthreads();
+  const int rp = (int)blockIdx.x * G + (int)threadIdx.x / TPT;
+  const bool active = rp < ny / 2;
+  const int y0 = active ? 2 * rp : 0;
+  cplx<T>* L = lds + ((int)threadIdx.x / TPT) * (2 * NX);
+  // inverse transform of rows y0, y0 + 1 of mixed field f: row y0 = Re, row y0 + 1 = -Im
+  auto inverse_rows = [&](const cplx<T>* f, cplx<T> (&w)[1][P]) {
+    cplx<T> A[P], B[P];
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      // every lane loads a valid element and a select clears what it must not use (herm_load)
+      const int k = t + TPT * q, kk = k <= nx / 2 ? k : nx - k;
+      const int kc = kk < 0 || a.kin <= 0 ? 0 : (kk < a.kin ? kk : a.kin - 1);
+      A[q] = at(f, boff32(kc, y0, ny));
+      B[q] = at(f, boff32(kc, y0 + 1, ny));
+    }
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const int k = t + TPT * q, kk = k <= nx / 2 ? k : nx - k;
+      const bool ok = k < nx && kk < a.kin, real = kk == 0 || 2 * kk == nx, up = 2 * k > nx;
+      const T ai = real ? (T)0 : (up ? -A[q].im : A[q].im), bi = real ? (T)0 : (up ? -B[q].im : B[q].im);
+      w[0][q] = ok ? mk(A[q].re - bi, -(ai + B[q].re)) : czero<T>();     // conj(A + i B)
+    }
+    dft_even<T, NX, P>(w, L, t, nx, tw);
   };
+  // forward transform of (row y0 + i row y0 + 1), split into the two rows' kept columns
+  auto forward_split = [&](cplx<T> (&w)[1][P], cplx<T> (&r0)[MAXI], cplx<T> (&r1)[MAXI]) {
+    dft_even<T, NX, P>(w, L, t, nx, tw);
+#pragma unroll
+    for (int q = 0; q < P; ++q) L[t + TPT * q] = w[0][q];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MAXI; ++i) {
+      const int kr = t + i * TPT;
+      if (kr < a.kout) {
+        const cplx<T> Wk = L[kr], Wm = L[kr == 0 ? 0 : nx - kr];
+        r0[i] = split_row(Wk, Wm, 0);
+        r1[i] = split_row(Wk, Wm, 1);
+      }
+    }
+    __syncthreads();
+  };
+  auto store = [&](cplx<T>* o, const cplx<T> (&r0)[MAXI], const cplx<T> (&r1)[MAXI]) {
+    if (!active) return;
+#pragma unroll
+    for (int i = 0; i < MAXI; ++i) {
+      const int kr = t + i * TPT;
+      if (kr < a.kout) {
+        at(o, boff32(kr, y0, ny)) = r0[i];
+        at(o, boff32(kr, y0 + 1, ny)) = r1[i];
+      }
+    }
+  };
+  cplx<T> w[1][P], r0[MAXI], r1[MAXI];
   if constexpr (MODE == K2_INVERSE_OUT) {
-    for (int f = 0; f < a.nfields; ++f) {
-      __syncthreads();
-      load(0, a.in + (long)f * a.fstride);
-      __syncthreads();
-      for (int x = t; x < nx; x += K2G_THREADS) a.phys[f * a.pstride + (long)y * nx + x] = c2r_point(S.hs[0], a.kin, nx, x, S.roots);
+    const long f = blockIdx.y;
+    inverse_rows(a.in + f * a.fstride, w);
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const int x = t + TPT * q;
+      if (!active || x >= nx) continue;
+      a.phys[f * a.pstride + (long)y0 * nx + x] = w[0][q].re;
+      a.phys[f * a.pstride + (long)(y0 + 1) * nx + x] = -w[0][q].im;
     }
   } else if constexpr (MODE == K2_FORWARD_IN) {
-    for (int f = 0; f < a.nfields; ++f) {
-      __syncthreads();
-      for (int x = t; x < nx; x += K2G_THREADS) S.ph[0][x] = a.phys_in[f * a.pstride + (long)y * nx + x];
-      __syncthreads();
-      cplx<T>* o = a.out + (long)f * a.ostride;
-      for (int kr = t; kr < a.kout; kr += K2G_THREADS) at(o, boff32(kr, y, ny)) = r2c_point(S.ph[0], nx, kr, S.roots);
+    const long f = blockIdx.y;
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const int x = t + TPT * q;
+      w[0][q] = x < nx ? mk(a.phys_in[f * a.pstride + (long)y0 * nx + x], a.phys_in[f * a.pstride + (long)(y0 + 1) * nx + x]) : czero<T>();
     }
+    forward_split(w, r0, r1);
+    store(a.out + f * a.ostride, r0, r1);
   } else {
-    // K2_ADVECT: u (q [+ eta]), v (q [+ eta]) (src/twodnavierstokes.jl:262-270,
-    // src/singlelayerqg.jl:368-375); K2_ADVECT_FULL, per layer: u += U,
-    // (-i kr (u q)^ - (u Qx + v Qy)^, (v q)^) (src/multilayerqg.jl:695-731), or with `linear`
-    // U q in place of u q and no v q (src/multilayerqg.jl:744-779)
+    // K2_ADVECT: u (q [+ eta]) in workgroup row 0, v (q [+ eta]) in row 1 (src/twodnavierstokes.jl:262-270,
+    // src/singlelayerqg.jl:368-375); K2_ADVECT_FULL, one layer per workgroup row: u += U,
+    // (-i kr (u q)^ - (u Qx + v Qy)^, (v q)^) (src/multilayerqg.jl:695-731), or with `linear` U q in place of
+    // u q and no v q (src/multilayerqg.jl:744-779)
     constexpr bool FULL = MODE == K2_ADVECT_FULL;
-    const int nl = FULL ? g.nlayers : 1;
-    for (int jl = 0; jl < nl; ++jl) {
-      __syncthreads();
-      for (int s = 0; s < 3; ++s) load(s, a.in + (long)(3 * jl + s) * a.fstride);
-      __syncthreads();
-      for (int x = t; x < nx; x += K2G_THREADS) {
-        T u = c2r_point(S.hs[0], a.kin, nx, x, S.roots);
-        const T v = c2r_point(S.hs[1], a.kin, nx, x, S.roots);
-        T q = c2r_point(S.hs[2], a.kin, nx, x, S.roots);
-        if constexpr (!FULL) {
-          if (a.eta != nullptr) q = q + a.eta[(long)y * nx + x];
-          S.ph[0][x] = u * q;
-          S.ph[1][x] = v * q;
-        } else {
-          T c = 0, U = 0;
-          if (a.has_bg) {
-            U = a.Uy[jl * ny + y];
-            u = u + U;
-            T qy = a.Qy1[jl * ny + y], qx = 0;
-            if (jl == nl - 1) {
-              if (a.etax) qx = a.etax[(long)y * nx + x];
-              if (a.etay) qy = qy + a.etay[(long)y * nx + x];
-            }
-            c = u * qx + v * qy;
+    const int jl = FULL ? (int)blockIdx.y : 0, half = FULL ? 0 : (int)blockIdx.y;
+    const cplx<T>* in = a.in + (long)(3 * jl) * a.fstride;
+    cplx<T>* out = a.out + (long)(2 * jl) * a.ostride;
+    T q0[P], q1[P];
+    inverse_rows(in + 2 * a.fstride, w);
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      q0[q] = w[0][q].re;
+      q1[q] = -w[0][q].im;
+      const int x = t + TPT * q;
+      if (!FULL && a.eta != nullptr && x < nx) {
+        q0[q] = q0[q] + a.eta[(long)y0 * nx + x];
+        q1[q] = q1[q] + a.eta[(long)(y0 + 1) * nx + x];
+      }
+    }
+    inverse_rows(in + (half ? a.fstride : 0), w);
+    if constexpr (!FULL) {
+#pragma unroll
+      for (int q = 0; q < P; ++q) w[0][q] = mk(w[0][q].re * q0[q], -w[0][q].im * q1[q]);
+      forward_split(w, r0, r1);
+      store(out + (half ? a.ostride : 0), r0, r1);
+    } else {
+      T u0[P], u1[P];
+      cplx<T> zb[1][P], zc[1][P];
+#pragma unroll
+      for (int q = 0; q < P; ++q) { u0[q] = w[0][q].re; u1[q] = -w[0][q].im; }
+      inverse_rows(in + a.fstride, w);
+      const T U0 = a.has_bg ? a.Uy[jl * ny + y0] : (T)0, U1 = a.has_bg ? a.Uy[jl * ny + y0 + 1] : (T)0;
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        const int x = t + TPT * q;
+        const T v0 = w[0][q].re, v1 = -w[0][q].im;
+        T c0 = 0, c1 = 0;
+        if (a.has_bg) {
+          u0[q] = u0[q] + U0;
+          u1[q] = u1[q] + U1;
+          T qy0 = a.Qy1[jl * ny + y0], qy1 = a.Qy1[jl * ny + y0 + 1], qx0 = 0, qx1 = 0;
+          if (jl == g.nlayers - 1 && x < nx) {
+            if (a.etax) { qx0 = a.etax[(long)y0 * nx + x]; qx1 = a.etax[(long)(y0 + 1) * nx + x]; }
+            if (a.etay) { qy0 = qy0 + a.etay[(long)y0 * nx + x]; qy1 = qy1 + a.etay[(long)(y0 + 1) * nx + x]; }
           }
-          S.ph[0][x] = a.linear ? U * q : u * q;
-          S.ph[1][x] = a.linear ? (T)0 : v * q;
-          S.ph[2][x] = c;
+          c0 = u0[q] * qx0 + v0 * qy0;
+          c1 = u1[q] * qx1 + v1 * qy1;
         }
+        zc[0][q] = mk(c0, c1);
+        zb[0][q] = a.linear ? czero<T>() : mk(v0 * q0[q], v1 * q1[q]);
+        w[0][q] = a.linear ? mk(U0 * q0[q], U1 * q1[q]) : mk(u0[q] * q0[q], u1[q] * q1[q]);
       }
-      __syncthreads();
-      cplx<T>* oA = a.out + (long)(FULL ? 2 * jl : 0) * a.ostride;
-      cplx<T>* oB = oA + a.ostride;
-      for (int kr = t; kr < a.kout; kr += K2G_THREADS) {
-        cplx<T> A = r2c_point(S.ph[0], nx, kr, S.roots);
-        const cplx<T> B = r2c_point(S.ph[1], nx, kr, S.roots);
-        if constexpr (FULL) {
-          const cplx<T> C = r2c_point(S.ph[2], nx, kr, S.roots);
-          const T kv = krwave(g, kr);
-          A = mk(kv * A.im - C.re, -kv * A.re - C.im);   // -i kr (u q)^ - (u Qx + v Qy)^
-        }
-        at(oA, boff32(kr, y, ny)) = A;
-        at(oB, boff32(kr, y, ny)) = B;
+      forward_split(w, r0, r1);
+      cplx<T> c0[MAXI], c1[MAXI];
+      forward_split(zc, c0, c1);
+#pragma unroll
+      for (int i = 0; i < MAXI; ++i) {
+        const T kv = krwave(g, t + i * TPT);
+        r0[i] = mk(kv * r0[i].im - c0[i].re, -kv * r0[i].re - c0[i].im);   // -i kr (u q)^ - (u Qx + v Qy)^
+        r1[i] = mk(kv * r1[i].im - c1[i].re, -kv * r1[i].re - c1[i].im);
       }
+      store(out, r0, r1);
+      forward_split(zb, r0, r1);
+      store(out + a.ostride, r0, r1);
     }
   }
 }
-template <typename T>
+template <typename T, int NX>
 void k2_gen(const K2Args<T>& a, hipStream_t s) {
-  const dim3 grid(a.g.ny), blk(K2G_THREADS);
+  constexpr int G = K2G<NX>::G;
+  const int rows = a.mode == K2_ADVECT ? 2 : (a.mode == K2_ADVECT_FULL ? a.g.nlayers : a.nfields);
+  if (rows <= 0) return;
+  const dim3 grid((a.g.ny / 2 + G - 1) / G, rows), blk(G * K2G<NX>::TPT);
   switch (a.mode) {
-    case K2_ADVECT: GF_LAUNCH((k2_gen_kernel<T, K2_ADVECT>), grid, blk, 0, s, a); break;
-    case K2_ADVECT_FULL: GF_LAUNCH((k2_gen_kernel<T, K2_ADVECT_FULL>), grid, blk, 0, s, a); break;
-    case K2_INVERSE_OUT: GF_LAUNCH((k2_gen_kernel<T, K2_INVERSE_OUT>), grid, blk, 0, s, a); break;
-    case K2_FORWARD_IN: GF_LAUNCH((k2_gen_kernel<T, K2_FORWARD_IN>), grid, blk, 0, s, a); break;
+    case K2_ADVECT: GF_LAUNCH((k2_gen_kernel<T, NX, K2_ADVECT>), grid, blk, 0, s, a); break;
+    case K2_ADVECT_FULL: GF_LAUNCH((k2_gen_kernel<T, NX, K2_ADVECT_FULL>), grid, blk, 0, s, a); break;
+    case K2_INVERSE_OUT: GF_LAUNCH((k2_gen_kernel<T, NX, K2_INVERSE_OUT>), grid, blk, 0, s, a); break;
+    case K2_FORWARD_IN: GF_LAUNCH((k2_gen_kernel<T, NX, K2_FORWARD_IN>), grid, blk, 0, s, a); break;
     default: break;
   }
 }
@@ -1006,7 +1054,7 @@ __device__ __forceinline__ void k3_body(const K3Args<T>& a, int blk, cplx<T>* __
     const YMap<TPT> m(threadIdx.x);
     t = m.t;
     kr = 2 * (G == 1 ? pair_of_block(blk) : blk * G + m.slot) + m.c;
-    L = col_buffer<T, NY>(lds, m.slot, m.c);
+    L = col_buffer<T, YN<NY, GEN>::value>(lds, m.slot, m.c);
   } else {
     t = threadIdx.x;
     kr = single_column(blk);
@@ -1273,7 +1321,7 @@ template <int N, int NL, int CPW> struct K3Waves { static constexpr int value = 
 template <typename T, int NY, int P, int G, int NL, int CPW = 2, int EPI = -1, bool ML1 = false, bool GEN = false>
 __global__ __launch_bounds__(CPW * G * (NY / P)) __attribute__((amdgpu_waves_per_eu(K3Waves<NY, NL, CPW>::value)))
 void k3_kernel(const K3Args<T> a) {
-  __shared__ cplx<T> lds[CPW == 2 ? G * PairLds<T, NY>::value : LdsN<NY>::value];
+  __shared__ cplx<T> lds[CPW == 2 ? G * PairLds<T, YN<NY, GEN>::value>::value : LdsN<YN<NY, GEN>::value>::value];
   __shared__ cplx<T> tw[YTw<NY, P, GEN>::size];
   load_y_twiddles<T, NY, P, GEN>(tw, a.tw, a.g.ny);
   __syncthreads();
@@ -1314,6 +1362,8 @@ template <int N> struct PCand {
 };
 // Points per thread of the multi-layer y passes: 4 (more, shorter transforms) up to 2048, 8 at
 // 4096 (a column pair of 4096 points at 4 per thread would need 2048 threads)
+// (column lengths that are not powers of two: 4, as dft_even needs)
+constexpr int PGEN = 4;
 template <int N> struct PML { static constexpr int P = N >= 4096 ? 8 : (N >= 32 ? 4 : PY<N>::P); };
 
 template <typename T, int N, int NL, int P, bool GEN = false>
@@ -1327,7 +1377,7 @@ void k1_np(const K1Args<T>& a, hipStream_t s) {
     if (a.fieldset == FS_CALCN) GF_LAUNCH((k1_kernel<T, N, P, G, NL, M_MLQG, FS_CALCN, GEN>), grid, blk, 0, s, a);
     else if (a.fieldset == FS_OUT) GF_LAUNCH((k1_kernel<T, N, P, G, NL, M_MLQG, FS_OUT, GEN>), grid, blk, 0, s, a);
     else GF_LAUNCH((k1_kernel<T, N, P, G, NL, M_MLQG, FS_RAW, GEN>), grid, blk, 0, s, a);
-  } else if constexpr (P != PY<N>::P) {   // a tuned schedule: the calcN field set only
+  } else if constexpr (P != PY<N>::P && !GEN) {   // a tuned schedule: the calcN field set only
     if (a.model == M_TWODNS) GF_LAUNCH((k1_kernel<T, N, P, G, 1, M_TWODNS, FS_CALCN, GEN>), grid, blk, 0, s, a);
     else GF_LAUNCH((k1_kernel<T, N, P, G, 1, M_SLQG, FS_CALCN, GEN>), grid, blk, 0, s, a);
   } else {
@@ -1346,12 +1396,12 @@ template <typename T, int N, int NL>
 void k1_n(const K1Args<T>& a, hipStream_t s) {
   if constexpr (NL > 1) {
     if constexpr (N <= GEN_MAX) {
-      if (a.g.ny != N) { k1_np<T, N, NL, PML<N>::P, true>(a, s); return; }   // a column length below N
+      if (a.g.ny != N) { k1_np<T, N, NL, PGEN, true>(a, s); return; }   // a column length below N
     }
     k1_np<T, N, NL, PML<N>::P>(a, s);
   } else {
     if constexpr (N <= GEN_MAX) {
-      if (a.g.ny != N) { k1_np<T, N, 1, PY<N>::P, true>(a, s); return; }
+      if (a.g.ny != N) { k1_np<T, N, 1, PGEN, true>(a, s); return; }
     }
     const bool tuned = a.fieldset == FS_CALCN && a.p != 0 && a.p != PY<N>::P && PCand<N>::has(a.p);
     if (tuned && a.p == 4) { if constexpr (PCand<N>::has(4) && PY<N>::P != 4) { k1_np<T, N, 1, 4>(a, s); return; } }
@@ -1387,7 +1437,7 @@ void k2_np(const K2Args<T>& a, hipStream_t s) {
 template <typename T, int N, int NL>
 void k2_n(const K2Args<T>& a, hipStream_t s) {
   if constexpr (N <= GEN_MAX) {
-    if (a.g.nx != N) { k2_gen<T>(a, s); return; }   // a row length below N: direct sums
+    if (a.g.nx != N) { k2_gen<T, N>(a, s); return; }   // a row length below N
   }
   const bool tuned = NL == 1 && (a.mode == K2_ADVECT || a.mode == K2_ADVECT_FULL) && a.p != 0 &&
                      a.p != PY<N>::P && PCand<N>::has(a.p);
@@ -1414,7 +1464,7 @@ void k3_np(const K3Args<T>& a, hipStream_t s) {
     if (a.ncols > 0) GF_LAUNCH((k3_kernel<T, N, P, 1, NL, 1, -1, false, GEN>), dim3(nblk, a.lsplit ? NL : 1), dim3(N / P), 0, s, a);
     return;
   }
-  if constexpr (NL == 1 && P == PY<N>::P) {
+  if constexpr (NL == 1 && (GEN || P == PY<N>::P)) {
     if (a.model == M_MLQG) {   // one-layer MultiLayerQG: fixed schedule, column pairs
       const int nblk = pair_blocks(a.ncols, G);
       if (nblk > 0) GF_LAUNCH((k3_kernel<T, N, P, G, 1, 2, -1, true, GEN>), dim3(nblk), dim3(2 * G * (N / P)), 0, s, a);
@@ -1453,12 +1503,12 @@ template <typename T, int N, int NL>
 void k3_n(const K3Args<T>& a, hipStream_t s) {
   if constexpr (NL > 1) {
     if constexpr (N <= GEN_MAX) {
-      if (a.g.ny != N) { k3_np<T, N, NL, PML<N>::P, true>(a, s); return; }   // a column length below N
+      if (a.g.ny != N) { k3_np<T, N, NL, PGEN, true>(a, s); return; }   // a column length below N
     }
     k3_np<T, N, NL, PML<N>::P>(a, s);
   } else {
     if constexpr (N <= GEN_MAX) {
-      if (a.g.ny != N) { k3_np<T, N, 1, PY<N>::P, true>(a, s); return; }
+      if (a.g.ny != N) { k3_np<T, N, 1, PGEN, true>(a, s); return; }
     }
     const bool tuned = a.p != 0 && a.p != PY<N>::P && PCand<N>::has(a.p);
     if (tuned && a.p == 4) { if constexpr (PCand<N>::has(4) && PY<N>::P != 4) { k3_np<T, N, 1, 4>(a, s); return; } }
