@@ -32,6 +32,13 @@ template <typename T> __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T>
   return mk(a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re);
 }
 template <typename T> __device__ __forceinline__ cplx<T> rmul(T s, cplx<T> a) { return mk(s * a.re, s * a.im); }
+// s a + c, each part one fused operation
+template <typename T> __device__ __forceinline__ cplx<T> rfma(T s, cplx<T> a, cplx<T> c) {
+  return mk(__builtin_fma(s, a.re, c.re), __builtin_fma(s, a.im, c.im));
+}
+template <> __device__ __forceinline__ cplx<float> rfma(float s, cplx<float> a, cplx<float> c) {
+  return mk(__builtin_fmaf(s, a.re, c.re), __builtin_fmaf(s, a.im, c.im));
+}
 template <typename T> __device__ __forceinline__ cplx<T> conj(cplx<T> a) { return mk(a.re, -a.im); }
 // multiply by -i
 template <typename T> __device__ __forceinline__ cplx<T> mul_mi(cplx<T> a) { return mk(a.im, -a.re); }
@@ -66,13 +73,13 @@ template <typename T> __device__ __forceinline__ void dft8(cplx<T>* v) {
   cplx<T> o[4] = {v[1], v[3], v[5], v[7]};
   dft4(e); dft4(o);
   // o[k] *= w8^k
-  cplx<T> o1 = mk(h * (o[1].re + o[1].im), h * (o[1].im - o[1].re));
-  cplx<T> o2 = mul_mi(o[2]);
-  cplx<T> o3 = mk(h * (o[3].im - o[3].re), -h * (o[3].re + o[3].im));
-  v[0] = e[0] + o[0]; v[4] = e[0] - o[0];
-  v[1] = e[1] + o1;   v[5] = e[1] - o1;
-  v[2] = e[2] + o2;   v[6] = e[2] - o2;
-  v[3] = e[3] + o3;   v[7] = e[3] - o3;
+  const cplx<T> o1 = mk(o[1].re + o[1].im, o[1].im - o[1].re);    // times h
+  const cplx<T> o2 = mul_mi(o[2]);
+  const cplx<T> o3 = mk(o[3].im - o[3].re, -(o[3].re + o[3].im));   // times h
+  v[0] = e[0] + o[0];        v[4] = e[0] - o[0];
+  v[1] = rfma(h, o1, e[1]);  v[5] = rfma(-h, o1, e[1]);
+  v[2] = e[2] + o2;          v[6] = e[2] - o2;
+  v[3] = rfma(h, o3, e[3]);  v[7] = rfma(-h, o3, e[3]);
 }
 
 template <typename T> __device__ __forceinline__ void dft16(cplx<T>* v) {
@@ -232,14 +239,24 @@ __device__ __forceinline__ cplx<T>* col_buffer(cplx<T>* lds, int slot, int c) {
 // that are meant to stay in flight across the exchange. The "memory" clobber keeps the compiler
 // from moving memory accesses across it.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-template <bool LIGHT> __device__ __forceinline__ void xbarrier() {
-  if constexpr (LIGHT) lds_barrier();
-  else __syncthreads();
+// Barriers of the transforms' exchanges: X_FULL a __syncthreads, X_LDS lds_barrier, X_WAVE none at
+// all, for a transform held by lanes of one wave: a wave's LDS instructions execute in order, so
+// only the compiler must keep theirs.
+constexpr int X_FULL = 0, X_LDS = 1, X_WAVE = 2;
+template <int X> __device__ __forceinline__ void xbarrier() {
+  if constexpr (X == X_WAVE) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else if constexpr (X == X_LDS) {
+    lds_barrier();
+  } else {
+    __syncthreads();
+  }
 }
 
-// One Stockham pass (index PASS, stride NS) on C transforms, then recurse.  LIGHT: exchange
-// barriers without a memory fence (lds_barrier).
-template <typename T, int N, int P, int C, int PASS, int NS, bool LIGHT = false>
+// One Stockham pass (index PASS, stride NS) on C transforms, then recurse.  X: the exchanges'
+// barriers (xbarrier).
+template <typename T, int N, int P, int C, int PASS, int NS, int X = X_FULL>
 __device__ __forceinline__ void stockham(cplx<T> (&v)[C][P], cplx<T>* __restrict__ lds, int t,
                                          const cplx<T>* __restrict__ tw) {
   using PL = Plan<N, P>;
@@ -284,13 +301,13 @@ __device__ __forceinline__ void stockham(cplx<T> (&v)[C][P], cplx<T>* __restrict
 #pragma unroll
         for (int r = 0; r < R; ++r) wp[padg<G>(r * NS)] = v[c][b + r * M];
       }
-      xbarrier<LIGHT>();
+      xbarrier<X>();
       const cplx<T>* rp = lds + padg<G>(t);
 #pragma unroll
       for (int q = 0; q < P; ++q) v[c][q] = rp[padg<G>(TPT * q)];
-      xbarrier<LIGHT>();
+      xbarrier<X>();
     }
-    stockham<T, N, P, C, PASS + 1, NS * R, LIGHT>(v, lds, t, tw);
+    stockham<T, N, P, C, PASS + 1, NS * R, X>(v, lds, t, tw);
   }
 }
 
@@ -306,14 +323,14 @@ __device__ __forceinline__ void stockham(cplx<T> (&v)[C][P], cplx<T>* __restrict
 // (147 instead of 122), one wave per SIMD fewer.  Recomputing them costs a few integer
 // operations per pass, 1-5% of a kernel's time where the registers it frees do not let more
 // workgroups run at once, so kernels ask for it only at sizes where they do.
-template <typename T, int N, int P, int C, bool FRESH = false, bool LIGHT = false>
+template <typename T, int N, int P, int C, bool FRESH = false, int X = X_FULL>
 __device__ __forceinline__ void fft_forward(cplx<T> (&v)[C][P], cplx<T>* __restrict__ lds, int t,
                                             const cplx<T>* __restrict__ tw) {
   if constexpr (FRESH) {
     asm volatile("" : "+v"(t));
     __builtin_assume(t >= 0 && t < N / P);   // the asm hides t's range from the multiplies below
   }
-  stockham<T, N, P, C, 0, 1, LIGHT>(v, lds, t, tw);
+  stockham<T, N, P, C, 0, 1, X>(v, lds, t, tw);
 }
 
 // Transform of an even length n < N that is not a power of two, in the data layout of fft_forward
@@ -363,10 +380,10 @@ __device__ __forceinline__ void dft_even(cplx<T> (&v)[1][P], cplx<T>* __restrict
   for (int j = 0; j < jm; ++j) {
     const cplx<T> w = roots[idx];
     const cplx<T> E0 = eo[4 * j], O0 = eo[4 * j + 1], E1 = eo[4 * j + 2], O1 = eo[4 * j + 3];
-    c0 = c0 + rmul(w.re, E0);
-    d0 = d0 + rmul(w.im, O0);
-    c1 = c1 + rmul(w.re, E1);
-    d1 = d1 + rmul(w.im, O1);
+    c0 = rfma(w.re, E0, c0);
+    d0 = rfma(w.im, O0, d0);
+    c1 = rfma(w.re, E1, c1);
+    d1 = rfma(w.im, O1, d1);
     idx += k;
     if (idx >= m) idx -= m;                          // j k mod m
   }

@@ -110,7 +110,7 @@ struct K2Args {
   const T* etay;            // ny*nx, bottom layer, nullable
   int linear;               // MLQG linearised equations: advect q by U only
   int lsplit;               // multi-layer: one layer per workgroup row (blockIdx.y)
-  int hsplit;               // single-layer advection: row 0 forms u q, row 1 v q (blockIdx.y)
+  int hsplit;               // single-layer advection: 1 a thread group per field (k2_group_kernel), 2 staged
   int has_bg;               // any nonzero Qx/Qy/U term
   cplx<T>* out;             // flux (2 fields per layer) or mixed (forward-in)
   long ostride;

@@ -90,13 +90,17 @@ template <typename T> struct Coef {
   // elements i and i + 1 (every table carries 16 bytes of padding), the second then unused. With
   // a branch on the kind between a load and its use, the compiler waited for each coefficient
   // before issuing the next load.
-  __device__ __forceinline__ cplx<T> mul(uint32_t i, cplx<T> x) const {
+  __device__ __forceinline__ cplx<T> get(uint32_t i) const {
     const T* e = reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) +
                                             i * (uint32_t)(cplx_ ? sizeof(cplx<T>) : sizeof(T)));
-    const T re = e[0], im = e[1];
-    return cplx_ ? cmul(mk(re, im), x) : rmul(re, x);
+    return mk(e[0], e[1]);
   }
 };
+// c x and c x + y of a loaded coefficient
+template <typename T> __device__ __forceinline__ cplx<T> coef_mul(int cp, cplx<T> c, cplx<T> x) { return cp ? cmul(c, x) : rmul(c.re, x); }
+template <typename T> __device__ __forceinline__ cplx<T> coef_fma(int cp, cplx<T> c, cplx<T> x, cplx<T> y) {
+  return cp ? rfma(c.re, x, rfma(c.im, mk(-x.im, x.re), y)) : rfma(c.re, x, y);
+}
 
 // ---------------------------------------------------------------------------
 // K1: spectral state -> mixed fields (inverse y-transform), one column / group
@@ -176,6 +180,36 @@ template <bool GEN> __device__ __forceinline__ bool in_col(int l, int ny) {
   if constexpr (GEN) return l < ny; else return true;
 }
 
+// 1/|k|^2 (invKrsq, [FF] TwoDGrid: 0 at k = 0)
+template <typename T> __device__ __forceinline__ T inv_k2(int kr, int l, T kv, T lv) {
+  return (kr == 0 && l == 0) ? (T)0 : (T)1 / (kv * kv + lv * lv);
+}
+// SingleLayerQG psih (src/singlelayerqg.jl:484-490)
+template <typename T>
+__device__ __forceinline__ cplx<T> slqg_psi(int eb, T ell2inv, cplx<T> sv, int kr, int l, T kv, T lv) {
+  if (eb) {
+    const T d = (kv * kv + lv * lv) + ell2inv;
+    return mk(-sv.re / d, -sv.im / d);
+  }
+  return rmul(-inv_k2(kr, l, kv, lv), sv);
+}
+// Spectrum of the velocity (or psi) field `code` of a point's state sv: TwoDNS from iK = 1/|k|^2, the
+// QG models from psih = p
+template <typename T, int MODEL>
+__device__ __forceinline__ cplx<T> k1_field(int code, cplx<T> sv, T iK, cplx<T> p, T kv, T lv) {
+  if constexpr (MODEL == M_TWODNS) {
+    // uh = i l invK sol, vh = -i kr invK sol (src/twodnavierstokes.jl:254-255)
+    if (code == F_U) { const T aa = lv * iK; return mk(-aa * sv.im, aa * sv.re); }
+    if (code == F_V) { const T bb = kv * iK; return mk(bb * sv.im, -bb * sv.re); }
+    return rmul(-iK, sv);
+  } else {
+    // uh = -i l psih, vh = i kr psih (src/singlelayerqg.jl:360-361)
+    if (code == F_U) return mk(lv * p.im, -lv * p.re);
+    if (code == F_V) return mk(-kv * p.im, kv * p.re);
+    return p;
+  }
+}
+
 // Body of K1 for block blk of column pairs; lds holds 2G padded N-point buffers and
 // tw the per-pass twiddle tables (already loaded).
 template <typename T, int NY, int P, int G, int NL, int MODEL, int FS, bool GEN = false>
@@ -224,23 +258,20 @@ __device__ __forceinline__ void k1_body(const K1Args<T>& a, int blk, cplx<T>* __
       for (int q = 0; q < P; ++q) {
         const int l = t + TPT * q;
         const T lv = lwave(g, l);
-        const T K2 = kv * kv + lv * lv;
         if constexpr (MODEL == M_TWODNS) {
-          iK[q] = (kr == 0 && l == 0) ? (T)0 : (T)1 / K2;
+          iK[q] = inv_k2(kr, l, kv, lv);
         } else if constexpr (NL > 1) {
           cplx<T> acc = czero<T>();
           if (active && in_col<GEN>(l, ny)) {
             const T* mm = a.sinv + boff(kr, l, ny) * (NL * NL) + jl * NL;
 #pragma unroll
-            for (int k = 0; k < NL; ++k) acc = acc + rmul(mm[k], sval(k, l));
+            for (int k = 0; k < NL; ++k) acc = rfma(mm[k], sval(k, l), acc);
           }
           ps[q] = acc;
           // the bottom layer's psih, for K3's bottom drag of the same stage
           if (FS == FS_CALCN && jl == NL - 1 && a.psi_out != nullptr && active && in_col<GEN>(l, ny)) at(a.psi_out, boff32(kr, l, ny)) = acc;
         } else {
-          const cplx<T> sv = svs[q];
-          if (a.eb) ps[q] = mk(-sv.re / (K2 + a.ell2inv), -sv.im / (K2 + a.ell2inv));
-          else ps[q] = rmul(-((kr == 0 && l == 0) ? (T)0 : (T)1 / K2), sv);
+          ps[q] = slqg_psi(a.eb, a.ell2inv, svs[q], kr, l, kv, lv);
         }
       }
     }
@@ -269,21 +300,8 @@ __device__ __forceinline__ void k1_body(const K1Args<T>& a, int blk, cplx<T>* __
         const int l = t + TPT * q;
         const T lv = lwave(g, l);
         cplx<T> r;
-        if (code == F_RAW || code == F_Q) {
-          r = svs[q];
-        } else if constexpr (MODEL == M_TWODNS) {
-          // uh = i l invK sol, vh = -i kr invK sol (src/twodnavierstokes.jl:254-255)
-          const cplx<T> sv = svs[q];
-          if (code == F_U) { const T aa = lv * iK[q]; r = mk(-aa * sv.im, aa * sv.re); }
-          else if (code == F_V) { const T bb = kv * iK[q]; r = mk(bb * sv.im, -bb * sv.re); }
-          else { r = rmul(-iK[q], sv); }
-        } else {
-          // uh = -i l psih, vh = i kr psih (src/singlelayerqg.jl:360-361)
-          const cplx<T> p = ps[q];
-          if (code == F_U) r = mk(lv * p.im, -lv * p.re);
-          else if (code == F_V) r = mk(-kv * p.im, kv * p.re);
-          else r = p;
-        }
+        if (code == F_RAW || code == F_Q) r = svs[q];
+        else r = k1_field<T, MODEL>(code, svs[q], MODEL == M_TWODNS ? iK[q] : (T)0, ps[q], kv, lv);
         // normalised inverse = conj(F(conj(x)))/(nx ny); the scale is a power of two
         w[0][q] = mk(r.re * nrm, -(r.im * nrm));
       }
@@ -497,7 +515,8 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
         }
       }
     }
-    // with hsplit, workgroup row 0 forms u q and row 1 v q (each transforms q itself)
+    // with hsplit 1 where a thread group per field does not fit (K2P), workgroup row 0 forms u q and
+    // row 1 v q (each transforms q itself)
     const int half = a.hsplit == 1 ? (int)blockIdx.y : 2;
     if (half != 1) {
       cplx<T> w[1][P];
@@ -839,6 +858,182 @@ void k2_kernel(const K2Args<T> a) {
 }
 
 // ---------------------------------------------------------------------------
+// K2, grouped: one thread group per field
+// ---------------------------------------------------------------------------
+// Small grids leave the GPU idle and the x pass waiting for its own chain of transforms.  Here each
+// row pair has three thread groups: group 0 transforms u, group 1 v, group 2 q, all at once; the
+// physical rows cross groups through LDS once, and the forward transforms of the products run
+// side by side too, so the chain is two transforms deep instead of five (or three where the
+// products had a workgroup each, every one transforming q again).  With P chosen so that a group
+// is one wave, its exchanges need no barrier (X_WAVE).  The layers of a multi-layer problem are
+// workgroup rows.  FULL: advection with background gradients (k2_body's K2_ADVECT_FULL).
+// FP64 per launch, against the two workgroup rows of three transforms before: 64^2 5.2 -> 4.4 us, 128^2
+// 5.8 -> 4.6, 256^2 6.5 -> 4.7, 512^2 8.5 -> 7.0; MultiLayerQG 512^2 x 3, against a layer per workgroup row,
+// 17.4 -> 16.4.
+template <int NX, int P> struct K2P {
+  static constexpr int TPT = NX / P;
+  static constexpr int G = TPT >= 64 ? 1 : 64 / TPT;   // row pairs per group: whole waves
+  static constexpr int GT = G * TPT;                   // threads per group
+  static constexpr int X = GT == 64 ? X_WAVE : X_LDS;
+  static constexpr bool fits(int size) { return 3 * GT <= 1024 && 3 * G * LdsN<NX>::value * size <= 120 * 1024; }
+};
+template <typename T, int NX, int P, bool FULL>
+__global__ __launch_bounds__((3 * K2P<NX, P>::GT)) __attribute__((amdgpu_waves_per_eu(2)))
+void k2_group_kernel(const K2Args<T> a) {
+  using K = K2P<NX, P>;
+  constexpr int TPT = K::TPT, G = K::G, X = K::X, PG = XPad<T>::G;
+  constexpr int MAXI = (NX / 2 + 1 + TPT - 1) / TPT;
+  constexpr int QH = P / 2 + 1;                        // the q with TPT q <= NX/2
+  __shared__ cplx<T> lds[3 * G * LdsN<NX>::value];
+  __shared__ cplx<T> tw[TwPlan<NX, P>::size()];
+  const Geo<T>& g = a.g;
+  const int ny = g.ny;
+  const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x / K::GT);
+  const int t = (int)threadIdx.x % TPT, slot = ((int)threadIdx.x % K::GT) / TPT;
+  const int jl = (int)blockIdx.y;
+  const int rp = xcd_block(blockIdx.x, gridDim.x) * G + slot;
+  const bool active = rp < ny / 2;
+  const int y0 = 2 * rp;
+  auto buffer = [&](int f) { return lds + (f * G + slot) * LdsN<NX>::value; };
+  cplx<T>* L = buffer(grp);
+  cplx<T> w[1][P];
+  {
+    const cplx<T>* f = a.in + (long)(3 * jl + grp) * a.fstride;
+    cplx<T> A[QH], B[QH];
+#pragma unroll
+    for (int q = 0; q < QH; ++q) {
+      const int k = t + TPT * q;
+      A[q] = herm_load<T, NX>(f, k, y0, ny, a.kin, active && k <= NX / 2);
+      B[q] = herm_load<T, NX>(f, k, y0 + 1, ny, a.kin, active && k <= NX / 2);
+    }
+    load_twiddles<T, NX, P>(tw, a.tw);
+#pragma unroll
+    for (int q = 0; q < QH; ++q) {
+      const int k = t + TPT * q;
+      if (k > NX / 2) continue;
+      w[0][q] = mk(A[q].re - B[q].im, -(A[q].im + B[q].re));     // conj(A + i B)
+      if (k > 0 && k < NX / 2) L[padg<PG>(NX - k)] = mk(A[q].re + B[q].im, A[q].im - B[q].re);
+    }
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      if (TPT * q + TPT - 1 <= NX / 2) continue;      // every lane of this q holds k <= NX/2
+      const int k = t + TPT * q;
+      if (k <= NX / 2) continue;
+      w[0][q] = L[padg<PG>(k)];
+    }
+    xbarrier<X>();
+  }
+  fft_forward<T, NX, P, 1, false, X>(w, L, t, tw);     // row y0 = Re, row y0 + 1 = -Im
+#pragma unroll
+  for (int q = 0; q < P; ++q) w[0][q] = conj(w[0][q]);  // (row y0, row y0 + 1)
+  if (!FULL && grp == 2 && a.eta != nullptr && active) {
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const int x = t + TPT * q;
+      w[0][q] = mk(w[0][q].re + at(a.eta, (uint32_t)(y0 * NX + x)), w[0][q].im + at(a.eta, (uint32_t)((y0 + 1) * NX + x)));
+    }
+  }
+  if (FULL || grp == 2) {
+#pragma unroll
+    for (int q = 0; q < P; ++q) L[padg<PG>(t) + padg<PG>(TPT * q)] = w[0][q];
+  }
+  lds_barrier();
+  if constexpr (!FULL) {
+    if (grp == 2 && X == X_WAVE) return;               // (waves that share barriers stay)
+    const cplx<T>* Q = buffer(2) + padg<PG>(t);
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const cplx<T> qv = Q[padg<PG>(TPT * q)];
+      w[0][q] = mk(w[0][q].re * qv.re, w[0][q].im * qv.im);
+    }
+    if constexpr (X != X_WAVE) lds_barrier();          // group 2's buffer is read: it may transform along
+  } else {
+    // u += U; z = u q, v q, u Qx + v Qy (src/multilayerqg.jl:695-731); linearised: U q, -, u Qx + v Qy
+    // (src/multilayerqg.jl:744-779)
+    T U0 = 0, U1 = 0;
+    if (active && a.has_bg) { U0 = a.Uy[jl * ny + y0]; U1 = a.Uy[jl * ny + y0 + 1]; }
+    const int off = padg<PG>(t);
+    if (grp < 2) {
+      const cplx<T>* Q = buffer(2) + off;
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        const cplx<T> qv = Q[padg<PG>(TPT * q)];
+        const T p0 = grp == 0 ? (a.linear ? U0 : w[0][q].re + U0) : (a.linear ? (T)0 : w[0][q].re);
+        const T p1 = grp == 0 ? (a.linear ? U1 : w[0][q].im + U1) : (a.linear ? (T)0 : w[0][q].im);
+        w[0][q] = mk(p0 * qv.re, p1 * qv.im);
+      }
+    } else {
+      const cplx<T>* Ub = buffer(0) + off;
+      const cplx<T>* Vb = buffer(1) + off;
+      T qy0 = 0, qy1 = 0;
+      if (active && a.has_bg) { qy0 = a.Qy1[jl * ny + y0]; qy1 = a.Qy1[jl * ny + y0 + 1]; }
+      const bool topo = active && a.has_bg && jl == g.nlayers - 1;
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        const int x = t + TPT * q;
+        const cplx<T> u = Ub[padg<PG>(TPT * q)], v = Vb[padg<PG>(TPT * q)];
+        T x0 = 0, x1 = 0, e0 = qy0, e1 = qy1;
+        if (topo && a.etax) { x0 = a.etax[(long)y0 * NX + x]; x1 = a.etax[(long)(y0 + 1) * NX + x]; }
+        if (topo && a.etay) { e0 = e0 + a.etay[(long)y0 * NX + x]; e1 = e1 + a.etay[(long)(y0 + 1) * NX + x]; }
+        w[0][q] = mk((u.re + U0) * x0 + v.re * e0, (u.im + U1) * x1 + v.im * e1);
+      }
+    }
+    lds_barrier();                                     // the rows are read: the buffers are free
+  }
+  fft_forward<T, NX, P, 1, false, X>(w, L, t, tw);     // of (row y0 + i row y0 + 1)
+  const MirrorSlots<NX, TPT, PG> ms(t);
+#pragma unroll
+  for (int q = 0; q < P; ++q) L[ms.k(q)] = w[0][q];
+  xbarrier<X>();
+  cplx<T> r0[MAXI], r1[MAXI];
+#pragma unroll
+  for (int i = 0; i < MAXI; ++i) {
+    const int kr = t + i * TPT;
+    if (kr < a.kout) {
+      const cplx<T> Wk = L[ms.k(i)], Wm = L[ms.m(i)];
+      r0[i] = split_row(Wk, Wm, 0);
+      r1[i] = split_row(Wk, Wm, 1);
+    }
+  }
+  if constexpr (FULL) {
+    // the spectrum of C = u Qx + v Qy goes to group 0, which stores -i kr (u q)^ - C
+    xbarrier<X>();
+    if (grp == 2) {
+#pragma unroll
+      for (int i = 0; i < MAXI; ++i) {
+        const int kr = t + i * TPT;
+        if (kr < a.kout) { L[kr] = r0[i]; L[NX / 2 + 1 + kr] = r1[i]; }
+      }
+    }
+    lds_barrier();
+    if (grp == 0) {
+      const cplx<T>* C = buffer(2);
+#pragma unroll
+      for (int i = 0; i < MAXI; ++i) {
+        const int kr = t + i * TPT;
+        if (kr < a.kout) {
+          const T kv = krwave(g, kr);
+          const cplx<T> c0 = C[kr], c1 = C[NX / 2 + 1 + kr];
+          r0[i] = mk(kv * r0[i].im - c0.re, -kv * r0[i].re - c0.im);
+          r1[i] = mk(kv * r1[i].im - c1.re, -kv * r1[i].re - c1.im);
+        }
+      }
+    }
+  }
+  if (grp == 2 || !active) return;
+  cplx<T>* o = a.out + (long)(2 * jl + grp) * a.ostride;
+#pragma unroll
+  for (int i = 0; i < MAXI; ++i) {
+    const int kr = t + i * TPT;
+    if (kr < a.kout) {
+      at(o, boff32(kr, y0, ny)) = r0[i];
+      at(o, boff32(kr, y0 + 1, ny)) = r1[i];
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // K2, staged: the x pass of advection without background gradients, loads one field ahead
 // ---------------------------------------------------------------------------
 // Each workgroup walks row pairs rp, rp + gridDim.x, ...  A field's two rows reach LDS through
@@ -928,7 +1123,7 @@ __device__ __forceinline__ void staged_store(cplx<T>* o, cplx<T> (&w)[1][P], int
   constexpr int TPT = NX / P;
   constexpr int MAXI = (NX / 2 + 1 + TPT - 1) / TPT;
   constexpr bool FR = NX >= FreshFrom<T>::k2;
-  fft_forward<T, NX, P, 1, FR, true>(w, L, t, tw);
+  fft_forward<T, NX, P, 1, FR, X_LDS>(w, L, t, tw);
   const MirrorSlots<NX, TPT, XPad<T>::G> ms(t);
 #pragma unroll
   for (int q = 0; q < P; ++q) L[ms.k(q)] = w[0][q];
@@ -967,7 +1162,7 @@ __device__ __forceinline__ void k2_staged_body(const K2Args<T>& a, cplx<T>* __re
       dma_wait();
       staged_take<T, NX, P>(w, S, L, t, kin);
       stage_rows<T, NX, P>(fu, y0, ny, kin, S);
-      fft_forward<T, NX, P, 1, FR, true>(w, L, t, tw);
+      fft_forward<T, NX, P, 1, FR, X_LDS>(w, L, t, tw);
 #pragma unroll
       for (int q = 0; q < P; ++q) {
         const int x = t + TPT * q;
@@ -984,7 +1179,7 @@ __device__ __forceinline__ void k2_staged_body(const K2Args<T>& a, cplx<T>* __re
       dma_wait();
       staged_take<T, NX, P>(w, S, L, t, kin);
       stage_rows<T, NX, P>(fv, y0, ny, kin, S);
-      fft_forward<T, NX, P, 1, FR, true>(w, L, t, tw);
+      fft_forward<T, NX, P, 1, FR, X_LDS>(w, L, t, tw);
 #pragma unroll
       for (int q = 0; q < P; ++q) w[0][q] = mk(w[0][q].re * q0[q], -w[0][q].im * q1[q]);   // u q, both rows
       staged_store<T, NX, P>(a.out, w, y0, ny, a.kout, L, tw, t);
@@ -994,7 +1189,7 @@ __device__ __forceinline__ void k2_staged_body(const K2Args<T>& a, cplx<T>* __re
       dma_wait();
       staged_take<T, NX, P>(w, S, L, t, kin);
       if (rp + nwg < npairs) stage_rows<T, NX, P>(fq, 2 * (rp + nwg), ny, kin, S);
-      fft_forward<T, NX, P, 1, FR, true>(w, L, t, tw);
+      fft_forward<T, NX, P, 1, FR, X_LDS>(w, L, t, tw);
 #pragma unroll
       for (int q = 0; q < P; ++q) w[0][q] = mk(w[0][q].re * q0[q], -w[0][q].im * q1[q]);   // v q, both rows
       staged_store<T, NX, P>(a.out + a.ostride, w, y0, ny, a.kout, L, tw, t);
@@ -1037,6 +1232,186 @@ int k2_staged_blocks(int npairs) {
 // runs on XCD b mod 8), so the later reads of each 16 BW-byte piece of the blocked layout (one
 // row of the block) hit in that XCD's L2.
 __device__ __forceinline__ int single_column(int b) { return BW * (8 * (b / (8 * BW)) + b % 8) + (b / 8) % BW; }
+
+// Where the stage epilogue of one spectral point (kr, l) of a layer reads and writes.
+template <typename T> struct StagePoint {
+  int kr, l, ny;
+  uint32_t idx, ix, cf, ci;   // in a field; in the layer's field; in the filter; in the coefficient tables
+  // The stepper's coefficient tables and the filter depend on kr and Krsq only, so rows l and
+  // ny - l hold equal values: reading the lower row lets the mirrored point's read hit in
+  // cache and halves the tables' HBM traffic.
+  __device__ __forceinline__ StagePoint(const K3Args<T>& a, int kr_, int l_, int ny_, uint32_t lo)
+      : kr(kr_), l(l_), ny(ny_), idx(boff32(kr_, l_, ny_)), ix(lo + idx), cf(boff32(kr_, l_ <= ny_ / 2 ? l_ : ny_ - l_, ny_)),
+        ci(a.cl_layered ? ix : cf) {}
+};
+// What the stage reads of that point: the state and its history (x: s1; y, z: n1, n23, or the RK and AB3
+// accumulators), the coefficients and the filter.  Every lane of an active column has the point, and
+// the stages compute for every lane and store only where kept: loads under a branch on kept made the
+// compiler wait for each before issuing the next.
+template <typename T> struct StageIn { cplx<T> sol, x, y, z, k[4]; T filter; };
+template <typename T>
+__device__ __forceinline__ StageIn<T> stage_load(const K3Args<T>& a, int epi, const StagePoint<T>& p) {
+  StageIn<T> in{};
+  auto coef = [&](const void* c) { return Coef<T>{c, a.ccplx}.get(p.ci); };
+  in.sol = at(a.sol, p.ix);
+  switch (epi) {
+    case E_ETD3:
+      in.x = at(a.s1, p.ix); in.y = at(a.n1, p.ix); in.z = at(a.n23, p.ix);
+      in.k[0] = coef(a.c0); in.k[1] = coef(a.c1);
+      break;
+    case E_ETD1: case E_ETD2:
+      in.k[0] = coef(a.c0); in.k[1] = coef(a.c1);
+      break;
+    case E_ETD4:
+      in.y = at(a.n1, p.ix); in.z = at(a.n23, p.ix);
+      in.k[0] = coef(a.c2); in.k[1] = coef(a.c3); in.k[2] = coef(a.c4); in.k[3] = coef(a.c5);
+      if (a.filter) in.filter = at(a.filter, p.cf);
+      break;
+    case E_RK1:
+      in.k[0] = coef(a.c0);
+      break;
+    case E_RK2: case E_RK3: case E_RK4:
+      in.k[0] = coef(a.c0); in.x = at(a.s1, p.ix); in.y = at(a.racc, p.ix);
+      if (epi == E_RK4 && a.filter) in.filter = at(a.filter, p.cf);
+      break;
+    case E_FE:
+      in.k[0] = coef(a.c0);
+      if (a.filter) in.filter = at(a.filter, p.cf);
+      break;
+    case E_AB3:
+      in.k[0] = coef(a.c0); in.y = at(a.racc, p.ix);
+      if (!a.ab3_start) in.z = at(a.n1, p.ix);
+      if (a.filter) in.filter = at(a.filter, p.cf);
+      break;
+    default: break;
+  }
+  return in;
+}
+// N of one point from its transformed fluxes Av, Bv, then the stage `epi`.  Returns the state the
+// next calcN! reads there (what kept points store).  NEXT: the caller hands that state on itself, so the
+// ETDRK4 stages 2 and 3, whose state nothing else reads, do not store it.
+template <typename T, int NL, bool ML1, bool NEXT>
+__device__ __forceinline__ cplx<T> stage_point(const K3Args<T>& a, int epi, const StagePoint<T>& p, const StageIn<T>& in, bool kept,
+                                               int jl, T kv, T lv, cplx<T> Av, cplx<T> Bv, cplx<T> psin, const cplx<T>* noise, bool& bad) {
+  const int kr = p.kr, l = p.l, ny = p.ny, cp = a.ccplx;
+  const uint32_t idx = p.idx, ix = p.ix;
+  cplx<T> N;
+  if (a.apply_kr) {
+    // N = -i kr (u zeta)^ - i l (v zeta)^ (src/twodnavierstokes.jl:272)
+    N = mk(kv * Av.im + lv * Bv.im, -kv * Av.re - lv * Bv.re);
+  } else {
+    N = mk(Av.re + lv * Bv.im, Av.im - lv * Bv.re);
+  }
+  if (a.etah != nullptr) {
+    // N -= i kr U etah (src/singlelayerqg.jl:379)
+    const cplx<T> e = at(a.etah, idx);
+    const T cu = kv * a.Ueta;
+    N = mk(N.re + cu * e.im, N.im - cu * e.re);
+  }
+  if constexpr (NL > 1) {
+    if (a.drag_src != nullptr && jl == NL - 1) {
+      // bottom drag N_n += mu Krsq psih_n (src/multilayerqg.jl:658)
+      const T K2 = kv * kv + lv * lv;
+      N = rfma(a.mu_drag * K2, psin, N);
+    }
+  }
+  if constexpr (ML1) {
+    if (a.drag_src != nullptr) {
+      // one layer: psih = -invKrsq qh of the (masked) calcN input, read before this point of
+      // the in-place stages is written; N += mu Krsq psih
+      const T K2 = kv * kv + lv * lv;
+      const cplx<T> ps = kept ? rmul(-inv_k2(kr, l, kv, lv), at(a.drag_src, ix)) : czero<T>();
+      N = rfma(a.mu_drag * K2, ps, N);
+    }
+  }
+  if (a.Fh != nullptr) N = rfma(a.fscale, at(a.Fh, ix), N);
+  if (a.sqrt_spec != nullptr) {
+    if (kr <= a.fkx && (l <= a.fky || l >= ny - a.fky)) {
+      if (at(a.sqrt_spec, idx) != (T)0) N = N + noise[kr * a.nbl + ring_box_row(l, ny, a.fky, a.nbl)];
+    }
+  }
+  const cplx<T> sv = kept ? in.sol : czero<T>();
+  if (a.nsave != nullptr) at(a.nsave, ix) = N;
+  cplx<T> r = czero<T>();
+  switch (epi) {
+    case E_CALCN:
+      at(a.nout, ix) = N;
+      break;
+    case E_ETD1:    // sol1 = E2 sol + zeta N1
+      r = coef_fma(cp, in.k[0], sv, coef_mul(cp, in.k[1], N));
+      if (kept) at(a.s1, ix) = r;
+      at(a.n1, ix) = N;
+      break;
+    case E_ETD2:    // sol2 = E2 sol + zeta N2
+      r = coef_fma(cp, in.k[0], sv, coef_mul(cp, in.k[1], N));
+      if (kept && !NEXT) at(a.s2, ix) = r;
+      at(a.n23, ix) = N;
+      break;
+    case E_ETD3:    // sol2 = E2 sol1 + zeta (2 N3 - N1)
+      r = coef_fma(cp, in.k[0], in.x, coef_mul(cp, in.k[1], mk((T)2 * N.re - in.y.re, (T)2 * N.im - in.y.im)));
+      if (kept && !NEXT) at(a.s2, ix) = r;
+      at(a.n23, ix) = in.z + N;
+      break;
+    case E_ETD4:    // sol = E sol + alpha N1 + 2 beta (N2 + N3) + Gamma N4
+      r = coef_fma(cp, in.k[1], in.y, coef_mul(cp, in.k[0], sv));
+      r = coef_fma(cp, in.k[2], mk((T)2 * in.z.re, (T)2 * in.z.im), r);
+      r = coef_fma(cp, in.k[3], N, r);
+      if (a.filter) r = rmul(in.filter, r);
+      at(a.sol_out != nullptr ? a.sol_out : a.sol, ix) = r;
+      bad |= !finite(r);
+      break;
+    case E_RK1:
+    case E_RK2:
+    case E_RK3:
+    case E_RK4: {
+      const cplx<T> xin = (epi == E_RK1) ? sv : (kept ? in.x : czero<T>());
+      const cplx<T> R = coef_fma(cp, in.k[0], xin, N);   // RHS = N + L sol_i
+      if (epi == E_RK1) {
+        r = rfma(a.dt / (T)2, R, sv);
+        if (kept) at(a.s1, ix) = r;
+        at(a.racc, ix) = mk(R.re / (T)6, R.im / (T)6);
+      } else if (epi == E_RK2) {
+        r = rfma(a.dt / (T)2, R, sv);
+        if (kept) at(a.s1, ix) = r;
+        at(a.racc, ix) = mk(in.y.re + R.re / (T)3, in.y.im + R.im / (T)3);
+      } else if (epi == E_RK3) {
+        r = rfma(a.dt, R, sv);
+        if (kept) at(a.s1, ix) = r;
+        at(a.racc, ix) = mk(in.y.re + R.re / (T)3, in.y.im + R.im / (T)3);
+      } else {
+        const cplx<T> acc = mk(in.y.re + R.re / (T)6, in.y.im + R.im / (T)6);
+        r = rfma(a.dt, acc, sv);
+        if (a.filter) r = rmul(in.filter, r);
+        at(a.sol, ix) = r;
+        bad |= !finite(r);
+      }
+    } break;
+    case E_FE:
+      r = rfma(a.dt, coef_fma(cp, in.k[0], sv, N), sv);
+      if (a.filter) r = rmul(in.filter, r);
+      at(a.sol, ix) = r;
+      bad |= !finite(r);
+      break;
+    case E_AB3: {
+      // RHS = N + L sol; forward Euler start-up, then 23/12 RHS - 16/12 RHS_1 + 5/12 RHS_2;
+      // the history (racc = RHS_1, n1 = RHS_2) shifts every step ([FF] AB3TimeStepper)
+      const cplx<T> R = coef_fma(cp, in.k[0], sv, N);
+      if (a.ab3_start) {
+        r = rfma(a.dt, R, sv);
+      } else {
+        const cplx<T> acc = rfma((T)(5.0 / 12.0), in.z, rfma(-(T)(16.0 / 12.0), in.y, rmul((T)(23.0 / 12.0), R)));
+        r = rfma(a.dt, acc, sv);
+      }
+      if (a.filter) r = rmul(in.filter, r);
+      at(a.sol, ix) = r;
+      at(a.n1, ix) = in.y;
+      at(a.racc, ix) = R;
+      bad |= !finite(r);
+    } break;
+    default: break;
+  }
+  return kept ? r : czero<T>();
+}
 
 // Body of K3 for block blk of column pairs (CPW = 2, G pairs per workgroup) or, with CPW = 1,
 // for the single column single_column(blk) (G = 1).  EPI >= 0 fixes the stage epilogue at
@@ -1115,7 +1490,7 @@ __device__ __forceinline__ void k3_body(const K3Args<T>& a, int blk, cplx<T>* __
   // stage 3, RK4 stages 2-3), so psi_n is formed before any layer is written.
   // With one layer per workgroup (lsplit), K1 of the same stage has stored it (psi_in): a
   // workgroup of another layer may already have overwritten that layer's input.
-  cplx<T> psin[P];
+  cplx<T> psin[NL > 1 ? P : 1];
   const int jl0 = (NL > 1 && a.lsplit) ? (int)blockIdx.y : 0;
   const int jl1 = (NL > 1 && a.lsplit) ? jl0 + 1 : NL;
   if constexpr (NL > 1) {
@@ -1131,7 +1506,7 @@ __device__ __forceinline__ void k3_body(const K3Args<T>& a, int blk, cplx<T>* __
           } else {
             const T* m = a.sinv + idx * (NL * NL) + (NL - 1) * NL;
 #pragma unroll
-            for (int k = 0; k < NL; ++k) ps = ps + rmul(m[k], a.drag_src[k * g.lstride + idx]);
+            for (int k = 0; k < NL; ++k) ps = rfma(m[k], a.drag_src[k * g.lstride + idx], ps);
           }
         }
         psin[q] = ps;
@@ -1159,147 +1534,9 @@ __device__ __forceinline__ void k3_body(const K3Args<T>& a, int blk, cplx<T>* __
       if (!in_col<GEN>(l, ny)) continue;
       const bool kept = (kept_l(g, l) && kr < g.kmax) || ((NL > 1 || ML1) && a.nomask);
       if (!kept && !a.full) continue;
-      const T lv = lwave(g, l);
-      const uint32_t idx = boff32(kr, l, ny);
-      const uint32_t ix = (uint32_t)lo + idx;
-      cplx<T> N;
-      const cplx<T> Av = A[0][q], Bv = B[0][q];
-      if (a.apply_kr) {
-        // N = -i kr (u zeta)^ - i l (v zeta)^ (src/twodnavierstokes.jl:272)
-        N = mk(kv * Av.im + lv * Bv.im, -kv * Av.re - lv * Bv.re);
-      } else {
-        N = mk(Av.re + lv * Bv.im, Av.im - lv * Bv.re);
-      }
-      if (a.etah != nullptr) {
-        // N -= i kr U etah (src/singlelayerqg.jl:379)
-        const cplx<T> e = at(a.etah, idx);
-        const T cu = kv * a.Ueta;
-        N = mk(N.re + cu * e.im, N.im - cu * e.re);
-      }
-      if constexpr (NL > 1) {
-        if (a.drag_src != nullptr && jl == NL - 1) {
-          // bottom drag N_n += mu Krsq psih_n (src/multilayerqg.jl:658)
-          const T K2 = kv * kv + lv * lv;
-          N = N + rmul(a.mu_drag * K2, psin[q]);
-        }
-      }
-      if constexpr (ML1) {
-        if (a.drag_src != nullptr) {
-          // one layer: psih = -invKrsq qh of the (masked) calcN input, read before this point of
-          // the in-place stages is written; N += mu Krsq psih
-          const T K2 = kv * kv + lv * lv;
-          const T iK = (kr == 0 && l == 0) ? (T)0 : (T)1 / K2;
-          const cplx<T> ps = kept ? rmul(-iK, at(a.drag_src, ix)) : czero<T>();
-          N = N + rmul(a.mu_drag * K2, ps);
-        }
-      }
-      if (a.Fh != nullptr) N = N + rmul(a.fscale, at(a.Fh, ix));
-      if (a.sqrt_spec != nullptr) {
-        if (kr <= a.fkx && (l <= a.fky || l >= ny - a.fky)) {
-          if (at(a.sqrt_spec, idx) != (T)0) N = N + noise[kr * a.nbl + ring_box_row(l, ny, a.fky, a.nbl)];
-        }
-      }
-      // The stepper's coefficient tables and the filter depend on kr and Krsq only, so rows l and
-      // NY - l hold equal values: reading the lower row lets the mirrored point's read hit in
-      // cache and halves the tables' HBM traffic.
-      const uint32_t cf = boff32(kr, l <= ny / 2 ? l : ny - l, ny);
-      const uint32_t ci = a.cl_layered ? ix : cf;
-      const cplx<T> svr = at(a.sol, ix);     // every lane of an active column has this point
-      const cplx<T> sv = kept ? svr : czero<T>();
-      if (a.nsave != nullptr) at(a.nsave, ix) = N;
-      switch (epi) {
-        case E_CALCN:
-          at(a.nout, ix) = N;
-          break;
-        // The stages compute for every lane and store only where kept: loads under a branch on
-        // kept made the compiler wait for each before issuing the next.
-        case E_ETD1: {  // sol1 = E2 sol + zeta N1
-          const Coef<T> E2{a.c0, a.ccplx}, Z{a.c1, a.ccplx};
-          const cplx<T> r = E2.mul(ci, sv) + Z.mul(ci, N);
-          if (kept) at(a.s1, ix) = r;
-          at(a.n1, ix) = N;
-        } break;
-        case E_ETD2: {  // sol2 = E2 sol + zeta N2
-          const Coef<T> E2{a.c0, a.ccplx}, Z{a.c1, a.ccplx};
-          const cplx<T> r = E2.mul(ci, sv) + Z.mul(ci, N);
-          if (kept) at(a.s2, ix) = r;
-          at(a.n23, ix) = N;
-        } break;
-        case E_ETD3: {  // sol2 = E2 sol1 + zeta (2 N3 - N1)
-          const Coef<T> E2{a.c0, a.ccplx}, Z{a.c1, a.ccplx};
-          const cplx<T> s1v = at(a.s1, ix);
-          const cplx<T> n1v = at(a.n1, ix);
-          const cplx<T> n23v = at(a.n23, ix);
-          const cplx<T> r = E2.mul(ci, s1v) + Z.mul(ci, mk((T)2 * N.re - n1v.re, (T)2 * N.im - n1v.im));
-          if (kept) at(a.s2, ix) = r;
-          at(a.n23, ix) = n23v + N;
-        } break;
-        case E_ETD4: {  // sol = E sol + alpha N1 + 2 beta (N2 + N3) + Gamma N4
-          const Coef<T> E{a.c2, a.ccplx}, Al{a.c3, a.ccplx}, Be{a.c4, a.ccplx}, Ga{a.c5, a.ccplx};
-          const cplx<T> n23v = at(a.n23, ix);
-          cplx<T> r = E.mul(ci, sv) + Al.mul(ci, at(a.n1, ix));
-          r = r + Be.mul(ci, mk((T)2 * n23v.re, (T)2 * n23v.im));
-          r = r + Ga.mul(ci, N);
-          if (a.filter) r = rmul(at(a.filter, cf), r);
-          at(a.sol_out != nullptr ? a.sol_out : a.sol, ix) = r;
-          bad |= !finite(r);
-        } break;
-        case E_RK1:
-        case E_RK2:
-        case E_RK3:
-        case E_RK4: {
-          const Coef<T> Lc{a.c0, a.ccplx};
-          const cplx<T> xin = (epi == E_RK1) ? sv : (kept ? at(a.s1, ix) : czero<T>());
-          const cplx<T> R = N + Lc.mul(ci, xin);   // RHS = N + L sol_i
-          if (epi == E_RK1) {
-            if (kept) at(a.s1, ix) = sv + rmul(a.dt / (T)2, R);
-            at(a.racc, ix) = mk(R.re / (T)6, R.im / (T)6);
-          } else if (epi == E_RK2) {
-            if (kept) at(a.s1, ix) = sv + rmul(a.dt / (T)2, R);
-            const cplx<T> ra = at(a.racc, ix);
-            at(a.racc, ix) = mk(ra.re + R.re / (T)3, ra.im + R.im / (T)3);
-          } else if (epi == E_RK3) {
-            if (kept) at(a.s1, ix) = sv + rmul(a.dt, R);
-            const cplx<T> ra = at(a.racc, ix);
-            at(a.racc, ix) = mk(ra.re + R.re / (T)3, ra.im + R.im / (T)3);
-          } else {
-            const cplx<T> ra = at(a.racc, ix);
-            const cplx<T> acc = mk(ra.re + R.re / (T)6, ra.im + R.im / (T)6);
-            cplx<T> r = sv + rmul(a.dt, acc);
-            if (a.filter) r = rmul(at(a.filter, cf), r);
-            at(a.sol, ix) = r;
-            bad |= !finite(r);
-          }
-        } break;
-        case E_FE: {
-          const Coef<T> Lc{a.c0, a.ccplx};
-          cplx<T> r = sv + rmul(a.dt, N + Lc.mul(ci, sv));
-          if (a.filter) r = rmul(at(a.filter, cf), r);
-          at(a.sol, ix) = r;
-          bad |= !finite(r);
-        } break;
-        case E_AB3: {
-          // RHS = N + L sol; forward Euler start-up, then 23/12 RHS - 16/12 RHS_1 + 5/12 RHS_2;
-          // the history (racc = RHS_1, n1 = RHS_2) shifts every step ([FF] AB3TimeStepper)
-          const Coef<T> Lc{a.c0, a.ccplx};
-          const cplx<T> R = N + Lc.mul(ci, sv);
-          const cplx<T> R1 = at(a.racc, ix);
-          cplx<T> r;
-          if (a.ab3_start) {
-            r = sv + rmul(a.dt, R);
-          } else {
-            const cplx<T> R2 = at(a.n1, ix);
-            const cplx<T> acc = (rmul((T)(23.0 / 12.0), R) - rmul((T)(16.0 / 12.0), R1)) + rmul((T)(5.0 / 12.0), R2);
-            r = sv + rmul(a.dt, acc);
-          }
-          if (a.filter) r = rmul(at(a.filter, cf), r);
-          at(a.sol, ix) = r;
-          at(a.n1, ix) = R1;
-          at(a.racc, ix) = R;
-          bad |= !finite(r);
-        } break;
-        default: break;
-      }
+      const StagePoint<T> pt(a, kr, l, ny, (uint32_t)lo);
+      const StageIn<T> in = stage_load<T>(a, epi, pt);
+      stage_point<T, NL, ML1, false>(a, epi, pt, in, kept, jl, kv, lwave(g, l), A[0][q], B[0][q], psin[NL > 1 ? q : 0], noise, bad);
       // With 8 points per thread, one point's loads and stores at a time keeps the epilogue
       // within 128 VGPRs (two 512-thread workgroups per CU) with less spilling than eight
       // points in flight; with 4 the registers allow all points' loads to be in flight at once.
@@ -1366,6 +1603,9 @@ template <int N> struct PCand {
 constexpr int PGEN = 4;
 template <int N> struct PML { static constexpr int P = N >= 4096 ? 8 : (N >= 32 ? 4 : PY<N>::P); };
 
+// ... and of their x pass
+template <int N> struct PMX { static constexpr int P = (N == 512 || N == 1024) ? 8 : 4; };
+
 template <typename T, int N, int NL, int P, bool GEN = false>
 void k1_np(const K1Args<T>& a, hipStream_t s) {
   constexpr int G = GY<N, P>::G;
@@ -1421,7 +1661,20 @@ void k2_np(const K2Args<T>& a, hipStream_t s) {
       return;
     }
   }
-  if constexpr (P != PY<N>::P) {          // a tuned schedule: the calcN modes only
+  if constexpr (K2P<N, P>::fits(sizeof(cplx<T>))) {
+    // a thread group per field: the split the schedule asks for, and every multi-layer problem
+    // (a layer per workgroup row) up to 1024 points
+    const bool full = a.mode == K2_ADVECT_FULL;
+    if (NL > 1 ? (full && a.lsplit && N <= 1024) : (a.hsplit == 1 && (full || a.mode == K2_ADVECT))) {
+      const dim3 gg((a.g.ny / 2 + K2P<N, P>::G - 1) / K2P<N, P>::G, NL), bb(3 * K2P<N, P>::GT);
+      if (full) GF_LAUNCH((k2_group_kernel<T, N, P, true>), gg, bb, 0, s, a);
+      else if constexpr (NL == 1) GF_LAUNCH((k2_group_kernel<T, N, P, false>), gg, bb, 0, s, a);
+      return;
+    }
+  }
+  if constexpr (NL > 1 && N <= 1024) {
+    return;                               // (multi-layer problems always have a layer per workgroup row)
+  } else if constexpr (P != PY<N>::P) {          // a tuned schedule: the calcN modes only
     if (a.mode == K2_ADVECT) { if constexpr (NL == 1) GF_LAUNCH((k2_kernel<T, N, P, G, K2_ADVECT, 1>), grid, blk, 0, s, a); }
     else GF_LAUNCH((k2_kernel<T, N, P, G, K2_ADVECT_FULL, NL>), grid, blk, 0, s, a);
   } else {
@@ -1448,9 +1701,8 @@ void k2_n(const K2Args<T>& a, hipStream_t s) {
   }
   (void)tuned;
   if constexpr (NL > 1) {
-    // multi-layer x pass: 4 points per thread (128-thread transforms at 512) -- one layer per
-    // workgroup row leaves the kernel latency-bound, and more threads per row pair shorten it
-    if (a.mode == K2_ADVECT_FULL && N >= 64) { k2_np<T, N, NL, 4>(a, s); return; }
+    // multi-layer x pass: a group of one wave per field up to 512 points
+    if (a.mode == K2_ADVECT_FULL && N >= 64) { k2_np<T, N, NL, PMX<N>::P>(a, s); return; }
   }
   k2_np<T, N, NL, PY<N>::P>(a, s);
 }
