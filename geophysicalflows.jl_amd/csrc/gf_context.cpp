@@ -862,14 +862,31 @@ struct Ctx final : CtxBase {
     }
   }
 
-  void calcN_launch(const C* in, int epi, bool full, const int64_t* fstep_dev = nullptr) {
+  void calcN_launch(const C* in, int epi, bool full) {
     K1Args<T> a; K2Args<T> b; K3Args<T> c;
     make_args(in, epi, full, a, b, c);
-    c.fstep_dev = fstep_dev;
     rec(0, true); launch_k1<T>(d.ny, a, stream); rec(0, false);
     rec(1, true); launch_k2<T>(d.nx, b, stream); rec(1, false);
     rec(2, true); launch_k3<T>(d.ny, c, stream); rec(2, false);
     HIPCHECK(hipGetLastError());
+  }
+  // The y passes of consecutive evaluations (K3 of one stage, K1 of the next) run as one launch where
+  // that kernel is built for the schedule: P and the columns per group as K3's, three groups per column
+  // where K1 has a field per workgroup row.  In the steps of such problems K1 too runs at K3's P, so
+  // that a step has the same bits whichever of its stages are fused (the first of a call, every
+  // stage while the kernels are timed one by one, and all under a split it is not built for, are not).
+  int ypass_p() const { return sched[2] ? sched[2] : sched_default(d.ny); }
+  bool ypass_fusable() const {
+    return tunable() && ystage_built(d.ny, ypass_p(), split[0] ? 3 : 1, split[2] && k3_single_column(d.ny, ypass_p()) ? 1 : 2);
+  }
+  // One stage of a run of stages on stream st: K1 unless the stage before has left its fields (first),
+  // the x pass, then K3 (last) or K3 with the next stage's K1.
+  void stage_launch(K1Args<T>& a, const K2Args<T>& b, const K3Args<T>& c, bool first, bool last, hipStream_t st) {
+    if (tunable()) a.p = ypass_p();
+    if (first) { rec(0, true); launch_k1<T>(d.ny, a, st); rec(0, false); }
+    rec(1, true); launch_k2<T>(d.nx, b, st); rec(1, false);
+    if (last) { rec(2, true); launch_k3<T>(d.ny, c, st); rec(2, false); }
+    else launch_ystage<T>(d.ny, c, a, st);
   }
 
   // the stages of one step: (calcN input, epilogue) pairs
@@ -1054,18 +1071,26 @@ struct Ctx final : CtxBase {
   // stage times of the configured stepper, as fractions of dt after the step's start
   // ([FF] ETDRK4 and RK4: t, t + dt/2, t + dt/2, t + dt; ForwardEuler and AB3: t)
   static double stage_offset(int k, int ns) { return ns == 1 ? 0.0 : (k == 0 ? 0.0 : (k == 3 ? 1.0 : 0.5)); }
-  void interior_launches(const int64_t* fstep_dev) {
+  // the stages of an interior step; fuse: its first stage's fields are there, and it leaves the next
+  // step's (stage_launch)
+  void interior_launches(const int64_t* fstep_dev, bool fuse) {
     const C* ins[4];
     int epis[4];
     const int ns = stages(ins, epis);
-    for (int k = 0; k < ns; ++k) calcN_launch(ins[k], epis[k], false, fstep_dev);
+    K1Args<T> a; K2Args<T> b; K3Args<T> c;
+    for (int k = 0; k < ns; ++k) {
+      make_args(ins[k], epis[k], false, a, b, c);
+      c.fstep_dev = fstep_dev;
+      stage_launch(a, b, c, !fuse, !fuse, stream);
+    }
+    HIPCHECK(hipGetLastError());
     if (fstep_dev) launch_counter(step_dev.as<int64_t>(), 1, 1, stream);
   }
   void build_graph(int which) {
     const bool ring = d.forcing == GF_FORCING_RING;
     if (ring && !step_dev.p) step_dev.alloc(sizeof(int64_t));
     gexec[which] = dw::capture(stream, [&] {
-      for (int s = 0; s < (which ? GRAPH_BLOCK : 1); ++s) interior_launches(ring ? step_dev.as<int64_t>() : nullptr);
+      for (int s = 0; s < (which ? GRAPH_BLOCK : 1); ++s) interior_launches(ring ? step_dev.as<int64_t>() : nullptr, ypass_fusable());
     });
   }
   void set_graphs(int enable) override { graphs = enable != 0; }
@@ -1075,6 +1100,9 @@ struct Ctx final : CtxBase {
     int epis[4];
     const int ns = stages(ins, epis);
     bool counter_set = false;
+    const bool fuse = ypass_fusable() && !tm.on;   // (the kernels are timed one by one)
+    bool fields = false;                           // the next stage's u, v, q are in the mixed fields
+    K1Args<T> ka; K2Args<T> kb; K3Args<T> kc;
     tm.mark(stream);
     for (int s = 0; s < n;) {
       const bool full = s == n - 1;
@@ -1094,6 +1122,12 @@ struct Ctx final : CtxBase {
           launch_counter(step_dev.as<int64_t>(), stepno, 0, stream);
           counter_set = true;
         }
+        if (fuse && !fields) {
+          make_args(ins[0], epis[0], false, ka, kb, kc);
+          ka.p = ypass_p();
+          launch_k1<T>(d.ny, ka, stream);
+          fields = true;
+        }
         HIPCHECK(hipGraphLaunch(gexec[which], stream));
         done = which ? GRAPH_BLOCK : 1;
       } else {
@@ -1102,8 +1136,12 @@ struct Ctx final : CtxBase {
             cur_fscale = (T)std::cos(f_omega * (t + stage_offset(k, ns) * d.dt) + f_phase);
             last_fscale = (double)cur_fscale;
           }
-          calcN_launch(ins[k], epis[k], full);
+          make_args(ins[k], epis[k], full, ka, kb, kc);
+          const bool last = !fuse || (full && k == ns - 1);
+          stage_launch(ka, kb, kc, !fields, last, stream);
+          fields = !last;
         }
+        HIPCHECK(hipGetLastError());
         cur_fscale = 1;
         counter_set = false;
       }
@@ -1484,26 +1522,29 @@ struct Ctx final : CtxBase {
   }
   void set_tape_budget(size_t bytes) override { tape_budget = bytes; }
 
-  // One ETDRK4 step from tape slot i (s0) writing N1..N4 of that slot and the new state to next
-  // (kept modes only: every later read masks), on stream st. The stage inputs s1, s2 and s3 (in
-  // s2's buffer, as in a plain step) go to the forward path's buffers, like the rest of its
-  // scratch (mixed, flux, n1, n23); the adjoint kernels use none of them.
-  void tape_step(long i, C* next, int tp, hipStream_t st) {
-    C* s0 = slot(i, 0, tp);
+  // n ETDRK4 steps from tape slot 0 (s0) of tape tp on stream st, writing N1..N4 of each step's slot and
+  // each new state to the next one (kept modes only: every later read masks). The stage inputs s1, s2
+  // and s3 (in s2's buffer, as in a plain step) go to the forward path's buffers, like the rest of
+  // its scratch (mixed, flux, n1, n23); the adjoint kernels use none of them.
+  void tape_steps(long n, int tp, hipStream_t st) {
     C* b1 = s1.as<C>();
     C* b2 = s2.as<C>();
+    const C* ins[4] = {nullptr, b1, b2, b2};
+    const int epis[4] = {E_ETD1, E_ETD2, E_ETD3, E_ETD4};
+    const bool fuse = ypass_fusable();
+    const bool was = tm.on;
+    tm.on = false;                         // (the sweep's own kernels are the timed ones)
     K1Args<T> a; K2Args<T> b; K3Args<T> k;
-    auto run = [&]() {
-      launch_k1<T>(d.ny, a, st); launch_k2<T>(d.nx, b, st); launch_k3<T>(d.ny, k, st);
-    };
-    make_args(s0, E_ETD1, false, a, b, k);
-    k.sol = s0; k.s1 = b1; k.nsave = slot(i, 1, tp); run();
-    make_args(b1, E_ETD2, false, a, b, k);
-    k.sol = s0; k.s2 = b2; k.nsave = slot(i, 2, tp); run();
-    make_args(b2, E_ETD3, false, a, b, k);
-    k.s1 = b1; k.s2 = b2; k.nsave = slot(i, 3, tp); run();
-    make_args(b2, E_ETD4, false, a, b, k);
-    k.sol = s0; k.sol_out = next; k.nsave = slot(i, 4, tp); k.nonfinite = nullptr; run();
+    for (long i = 0; i < n; ++i) {
+      C* s0 = slot(i, 0, tp);
+      for (int q = 0; q < 4; ++q) {
+        make_args(q == 0 ? s0 : ins[q], epis[q], false, a, b, k);
+        k.sol = s0; k.s1 = b1; k.s2 = b2; k.nsave = slot(i, q + 1, tp);
+        if (q == 3) { k.sol_out = slot(i + 1, 0, tp); k.nonfinite = nullptr; }
+        stage_launch(a, b, k, !fuse || (i == 0 && q == 0), !fuse || (i == n - 1 && q == 3), st);
+      }
+    }
+    tm.on = was;
     HIPCHECK(hipGetLastError());
   }
 
@@ -1615,7 +1656,7 @@ struct Ctx final : CtxBase {
                                 hipMemcpyDeviceToDevice, stream));
         HIPCHECK(hipMemcpyAsync(ckpts.as<C>() + s * kstride(), slot(0, 0, tp), kb, hipMemcpyDeviceToDevice, stream));
         const long n = len(s);
-        for (long i = 0; i < n; ++i) tape_step(i, slot(i + 1, 0, tp), tp, stream);
+        tape_steps(n, tp, stream);
       }
       // loss and lambda_T = M (w/N) rfft2(zeta_T - target), zeta_T = irfft2(M sol_T); the columns of
       // cinp past the tape's prefix hold stale values, which the mask clears
@@ -1653,7 +1694,7 @@ struct Ctx final : CtxBase {
         const int tp = tape_of(s);
         if (s < resident) {
           HIPCHECK(hipMemcpyAsync(slot(0, 0, tp), ckpts.as<C>() + s * kstride(), kb, hipMemcpyDeviceToDevice, stream));
-          for (long i = 0; i < n; ++i) tape_step(i, slot(i + 1, 0, tp), tp, stream);
+          tape_steps(n, tp, stream);
         }
         for (long i = n - 1; i >= 0; --i) adjoint_step(i, dnu != nullptr, tp);
       }
@@ -1666,7 +1707,7 @@ struct Ctx final : CtxBase {
           HIPCHECK(hipMemcpyAsync(slot(0, 0, tq), ckpts.as<C>() + (s - 1) * kstride(), kb, hipMemcpyDeviceToDevice,
                                   rstream));
           const long m = len(s - 1);
-          for (long i = 0; i < m; ++i) tape_step(i, slot(i + 1, 0, tq), tq, rstream);
+          tape_steps(m, tq, rstream);
           HIPCHECK(hipEventRecord(rec_done[tq], rstream));
         }
         if (s < resident) HIPCHECK(hipStreamWaitEvent(stream, rec_done[tp], 0));

@@ -288,6 +288,8 @@ template <typename T> void launch_pv_from_psi(const PvArgs<T>& a, hipStream_t s)
 template <typename T> void launch_k1(int ny, const K1Args<T>& a, hipStream_t s);
 template <typename T> void launch_k2(int nx, const K2Args<T>& a, hipStream_t s);
 template <typename T> void launch_k3(int ny, const K3Args<T>& a, hipStream_t s);
+// K3 of the stage c, then K1 (args a) of the next evaluation, on the same columns
+template <typename T> void launch_ystage(int ny, const K3Args<T>& c, const K1Args<T>& a, hipStream_t s);
 template <typename T> void launch_to_julia(const Geo<T>& g, const cplx<T>* src, cplx<T>* dst, int nl, hipStream_t s);
 template <typename T> void launch_from_julia(const Geo<T>& g, const cplx<T>* src, cplx<T>* dst, int nl, hipStream_t s);
 template <typename T> void launch_mask(const Geo<T>& g, cplx<T>* sol, int nl, hipStream_t s);
@@ -311,6 +313,14 @@ __host__ __device__ inline int ring_box_row(int l, int ny, int fky, int nbl) { r
 // K3 runs one column per workgroup (csplit) when a column's n/p threads fill at least one wave;
 // otherwise csplit is ignored and the column pairs share workgroups.
 constexpr bool k3_single_column(int n, int p) { return n / p >= 64; }
+// The fused y pass (gf_ystage_impl.hpp) that is built for columns of n points at p per thread with ng
+// thread groups per column: three (a field each) up to 1024 points where they fit a workgroup, one from 1024,
+// cpw = 1 or 2 columns per group.
+constexpr bool ystage_built(int n, int p, int ng, int cpw) {
+  if (n < 32 || n > 4096 || (cpw == 1 && !k3_single_column(n, p))) return false;
+  if (ng == 3) return n <= 1024 && (p == 4 || p == 8) && 3 * cpw * (n / p) <= 1024;
+  return n >= 1024 && ((p == 4 && n <= 2048) || p == 8 || (p == 16 && n == 4096));
+}
 // Workgroups of a launch with G column pairs per workgroup over ncols columns; with quads and
 // G = 1, a multiple of 16 (pair_of_block puts the two pairs of a block on one XCD).
 constexpr int pair_blocks(int ncols, int G) {

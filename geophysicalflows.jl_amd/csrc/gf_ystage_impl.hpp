@@ -1,0 +1,217 @@
+// The fused y pass of consecutive calcN! evaluations: K3 of one stage and K1 of the next.
+//
+// Both work on whole kr columns: K3 transforms a column's fluxes forward along y and steps its
+// modes, K1 reads those modes back, forms u, v and q and transforms them inversely.  Inside a
+// run of stages one kernel does both, so a stage is two launches (x pass, y pass) instead of
+// three, the new state is not read back, and the intermediate states of ETDRK4 that only the
+// next K1 reads (stages 2 and 3) are not written at all.  The first stage of a call starts with K1
+// and the last one ends with K3; every expression is the one those kernels evaluate
+// (stage_point, k1_field), so the results are theirs bit for bit.
+//
+// NG = 3: three thread groups per column (or column pairs).  Groups 0 and 1 transform the two fluxes
+// side by side, the modes of the column are stepped by all three, and each transforms one of u, v, q:
+// two transforms in a row where K3 and K1 run five.  Where a group is one wave the transforms need no
+// barriers (X_WAVE).  This serves the grids whose y passes wait on latency.
+// NG = 1: one group does all five, the state in registers in between: for grids that fill the GPU with
+// one group per column already.
+//
+// FP64 per launch, K3 + K1 -> fused: 64^2 5.8 + 3.4 -> 5.1 us, 128^2 6.6 + 3.6 -> 6.0, 512^2 10.3 + 6.1 -> 12.3,
+// 2048^2 (ETDRK4) 26.8 + 21.7 -> 39.6, where it moves 15% less than the two did.
+#include "gf_kernels_impl.hpp"
+
+namespace gf {
+
+template <int N, int P, int NG, int CPW> struct YS {
+  static constexpr int TPT = N / P;
+  static constexpr int G = CPW == 2 ? GY<N, P>::G : 1;
+  static constexpr int GT = CPW * G * TPT;             // threads per group, whole waves
+  static constexpr int X = GT == 64 ? X_WAVE : X_LDS;
+  static constexpr int QN = (P + NG - 1) / NG;         // modes a thread steps
+};
+template <typename T, int NY, int P, int NG, int CPW, int MODEL, int EPI>
+__global__ __launch_bounds__((NG * YS<NY, P, NG, CPW>::GT)) __attribute__((amdgpu_waves_per_eu(2)))
+void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
+  using Y = YS<NY, P, NG, CPW>;
+  constexpr int TPT = Y::TPT, G = Y::G, GT = Y::GT, X = Y::X, PG = XPad<T>::G;
+  constexpr int BUF = CPW == 2 ? G * PairLds<T, NY>::value : LdsN<NY>::value;
+  constexpr bool FR = NG == 1 && sizeof(T) == 8 && NY >= 2048;
+  __shared__ cplx<T> lds[NG * BUF];
+  __shared__ cplx<T> tw[TwPlan<NY, P>::size()];
+  const Geo<T>& g = c.g;
+  const int grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / GT);
+  const int tid = (int)threadIdx.x % GT;
+  int t, kr, col;
+  if constexpr (CPW == 2) {
+    const YMap<TPT> m(tid);
+    t = m.t;
+    kr = 2 * (G == 1 ? pair_of_block(blockIdx.x) : (int)blockIdx.x * G + m.slot) + m.c;
+    col = (int)(col_buffer<T, NY>(lds, m.slot, m.c) - lds);
+  } else {
+    t = tid;
+    kr = single_column(blockIdx.x);
+    col = 0;
+  }
+  cplx<T>* L = lds + grp * BUF + col;
+  const bool active = kr < c.ncols && kr < g.nkr;
+  const T kv = krwave(g, kr);
+  const int epi = EPI >= 0 ? EPI : c.epi;
+
+  // the fluxes of this column: group 0 (u q)^, group 1 (v q)^
+  cplx<T> w[1][P], w1[1][NG == 1 ? P : 1];
+  const int krl = active ? kr : 0;
+  {
+    const cplx<T>* f = c.in + (long)(grp == 1 ? c.fstride : 0);
+#pragma unroll
+    for (int q = 0; q < P; ++q) w[0][q] = at(f, boff32(krl, t + TPT * q, NY));
+    if constexpr (NG == 1) {
+#pragma unroll
+      for (int q = 0; q < P; ++q) w1[0][q] = at(c.in + c.fstride, boff32(krl, t + TPT * q, NY));
+    }
+  }
+  load_twiddles<T, NY, P>(tw, c.tw);
+  // what this thread's modes need from memory, under way during the transforms (NG = 3: two or three
+  // modes per thread; with one group the registers do not hold them)
+  auto row = [&](int i) { return t + TPT * (NG == 1 ? i : grp + NG * i); };
+  auto mine = [&](int i) { return NG == 1 || grp + NG * i < P; };
+  StageIn<T> in[NG == 1 ? 1 : Y::QN];
+  if constexpr (NG > 1) {
+#pragma unroll
+    for (int i = 0; i < Y::QN; ++i)
+      in[i] = stage_load<T>(c, epi, StagePoint<T>(c, krl, mine(i) ? row(i) : t, NY, 0u));
+  }
+  // ring forcing: this thread's terms, read back by it in the stage (k3_body)
+  if (c.sqrt_spec != nullptr && active && kr <= c.fkx) {
+    const int64_t fstep = c.fstep_dev != nullptr ? c.fstep_dev[0] : c.fstep;
+    for (int i = 0; i < Y::QN; ++i) {
+      const int l = row(i);
+      if (mine(i) && (l <= c.fky || l >= NY - c.fky)) {
+        const T sp = at(c.sqrt_spec, boff32(kr, l, NY));
+        if (sp != (T)0) {
+          const cplx<T> xi = complex_normal<T>(c.seed, fstep, (uint32_t)(l * g.nkr + kr), (uint32_t)c.instance);
+          c.noise[kr * c.nbl + ring_box_row(l, NY, c.fky, c.nbl)] = mk((xi.re * sp) / c.sqrt_dt, (xi.im * sp) / c.sqrt_dt);
+        }
+      }
+    }
+  }
+  lds_barrier();                                       // the twiddles
+  fft_forward<T, NY, P, 1, FR, X>(w, L, t, tw);
+  if constexpr (NG == 1) fft_forward<T, NY, P, 1, FR, X>(w1, L, t, tw);
+
+  bool bad = false;
+  cplx<T> sv[P];
+  if constexpr (NG == 1) {
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const int l = t + TPT * q;
+      const bool kept = kept_l(g, l) && kr < g.kmax;
+      sv[q] = czero<T>();
+      if (active && (kept || c.full)) {
+        const StagePoint<T> pt(c, kr, l, NY, 0u);
+        const StageIn<T> one = stage_load<T>(c, epi, pt);
+        sv[q] = stage_point<T, 1, false, true>(c, epi, pt, one, kept, 0, kv, lwave(g, l), w[0][q], w1[0][q], czero<T>(), c.noise, bad);
+      }
+      if constexpr (P >= 8) __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    // the transformed fluxes cross groups in buffers 0 and 1, the new modes come back in buffer 2
+    const int off = padg<PG>(t);
+    if (grp < 2) {
+#pragma unroll
+      for (int q = 0; q < P; ++q) L[off + padg<PG>(TPT * q)] = w[0][q];
+    }
+    lds_barrier();
+    const cplx<T>* A = lds + col;
+    const cplx<T>* B = lds + BUF + col;
+    cplx<T>* S = lds + 2 * BUF + col;
+#pragma unroll
+    for (int i = 0; i < Y::QN; ++i) {
+      if (!mine(i)) continue;
+      const int l = row(i), s = padg<PG>(l);
+      const bool kept = kept_l(g, l) && kr < g.kmax;
+      cplx<T> r = czero<T>();
+      if (active && (kept || c.full))
+        r = stage_point<T, 1, false, true>(c, epi, StagePoint<T>(c, kr, l, NY, 0u), in[i], kept, 0, kv, lwave(g, l), A[s], B[s], czero<T>(), c.noise, bad);
+      S[s] = r;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < P; ++q) sv[q] = S[off + padg<PG>(TPT * q)];
+    lds_barrier();                                     // buffer 2 is free
+  }
+  const unsigned long long badm = __ballot(bad);
+  if (badm != 0 && c.nonfinite != nullptr && (int)(threadIdx.x & 63) == __ffsll(badm) - 1) *c.nonfinite = 1;
+
+  // the next calcN!'s fields of the kept columns
+  const bool out = active && kr < a.ncols;
+  if (CPW == 1 && kr >= a.ncols) return;               // (a single column is its whole workgroup's)
+  T iK[P];
+  cplx<T> ps[P];
+#pragma unroll
+  for (int q = 0; q < P; ++q) {
+    const int l = t + TPT * q;
+    iK[q] = MODEL == M_TWODNS ? inv_k2(kr, l, kv, lwave(g, l)) : (T)0;
+    ps[q] = MODEL == M_TWODNS ? czero<T>() : slqg_psi(a.eb, a.ell2inv, sv[q], kr, l, kv, lwave(g, l));
+  }
+  const T nrm = g.inv_norm;
+#pragma unroll
+  for (int f = 0; f < (NG == 1 ? 3 : 1); ++f) {
+    const int field = NG == 1 ? f : grp;               // u, v, q (Fields<MODEL, FS_CALCN>)
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const T lv = lwave(g, t + TPT * q);
+      const cplx<T> r = field == 2 ? sv[q] : k1_field<T, MODEL>(field == 0 ? F_U : F_V, sv[q], iK[q], ps[q], kv, lv);
+      w[0][q] = mk(r.re * nrm, -(r.im * nrm));
+    }
+    fft_forward<T, NY, P, 1, FR, X>(w, L, t, tw);
+    if (out) {
+      cplx<T>* o = a.out + (long)field * a.fstride;
+#pragma unroll
+      for (int q = 0; q < P; ++q) at(o, boff32(kr, t + TPT * q, NY)) = conj(w[0][q]);
+    }
+  }
+}
+
+template <typename T, int N, int P, int NG, int CPW, int MODEL>
+void ystage_go(const K3Args<T>& c, const K1Args<T>& a, hipStream_t s) {
+  using Y = YS<N, P, NG, CPW>;
+  const int nblk = CPW == 1 ? column_blocks(c.ncols) : pair_blocks(c.ncols, Y::G);
+  if (c.ncols <= 0) return;
+  const dim3 grid(nblk), blk(NG * Y::GT);
+  if constexpr (NG == 1 && N >= 2048) {
+    // one kernel per ETDRK4 stage, as K3 has them: the stage's registers set the occupancy
+    switch (c.epi) {
+      case E_ETD1: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_ETD1>), grid, blk, 0, s, c, a); return;
+      case E_ETD2: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_ETD2>), grid, blk, 0, s, c, a); return;
+      case E_ETD3: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_ETD3>), grid, blk, 0, s, c, a); return;
+      case E_ETD4: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_ETD4>), grid, blk, 0, s, c, a); return;
+      default: break;
+    }
+  }
+  GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, -1>), grid, blk, 0, s, c, a);
+}
+template <typename T, int N, int P, int NG>
+void ystage_p(const K3Args<T>& c, const K1Args<T>& a, hipStream_t s) {
+  const bool twodns = c.model == M_TWODNS;
+  if constexpr (ystage_built(N, P, NG, 1)) {
+    if (c.csplit) {
+      if (twodns) ystage_go<T, N, P, NG, 1, M_TWODNS>(c, a, s);
+      else ystage_go<T, N, P, NG, 1, M_SLQG>(c, a, s);
+      return;
+    }
+  }
+  if constexpr (ystage_built(N, P, NG, 2)) {
+    if (twodns) ystage_go<T, N, P, NG, 2, M_TWODNS>(c, a, s);
+    else ystage_go<T, N, P, NG, 2, M_SLQG>(c, a, s);
+  }
+}
+template <typename T, int N, int NG>
+void ystage_n(const K3Args<T>& c, const K1Args<T>& a, hipStream_t s) {
+  switch (c.p ? c.p : sched_default(N)) {
+    case 4: ystage_p<T, N, 4, NG>(c, a, s); break;
+    case 8: ystage_p<T, N, 8, NG>(c, a, s); break;
+    case 16: ystage_p<T, N, 16, NG>(c, a, s); break;
+    default: break;
+  }
+}
+
+}  // namespace gf

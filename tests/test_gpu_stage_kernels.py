@@ -1,12 +1,16 @@
-"""The x pass with a thread group per field, at the edges of the sizes, radices and layouts it is built for.
+"""The x pass with a thread group per field and the y pass that fuses one stage's K3 with the next
+stage's K1, at the edges of the sizes, radices and layouts they are built for.
 
-Tolerances: the grouped x pass packs and transforms as the plain one and
+Tolerances: the fused y pass evaluates the expressions of K3 and K1, so it gives their bits (per-kernel
+timing steps with those two kernels).  The grouped x pass packs and transforms as the plain one and
 rounds differently at most: calcN agrees to the 1e-13 (FP64) and 2e-6 (FP32) that it is held to
 against the oracle.
 """
 import numpy as np
 import pytest
 
+from oracle import fourierflows as off
+from oracle import singlelayerqg as osl
 from tests.conftest import rel
 
 pytestmark = pytest.mark.gpu
@@ -35,3 +39,46 @@ def test_a_group_per_field_gives_the_plain_x_pass(gf, nx, ny, p2, dtype):
                 gf.set_splits(p, 0, k2, 0)
             out.append(p.calcN(s)[0])
         assert rel(out[1], out[0]) < tol
+
+
+# (nx, ny, P of K3, K1 split, K3 split): the smallest and largest columns of each form (three groups of one
+# and of several waves, one group, pairs and single columns) and rectangles
+FORMS = [(32, 32, 4, 1, 0), (32, 32, 8, 1, 0), (64, 64, 4, 1, 0), (128, 64, 8, 1, 0), (64, 128, 4, 1, 0), (32, 256, 4, 1, 1),
+         (256, 256, 8, 1, 0), (64, 512, 8, 1, 1), (64, 512, 4, 1, 0), (32, 1024, 4, 1, 1), (32, 1024, 8, 1, 0), (64, 1024, 8, 0, 1),
+         (32, 2048, 4, 0, 0), (64, 2048, 8, 0, 1), (32, 4096, 8, 0, 0), (32, 4096, 8, 0, 1), (32, 4096, 16, 0, 0)]
+
+
+@pytest.mark.parametrize("nx,ny,p3,k1,k3", FORMS)
+@pytest.mark.parametrize("stepper", ["ETDRK4", "FilteredRK4", "AB3", "FilteredForwardEuler"])
+def test_fused_stages_give_the_bits_of_the_separate_kernels(gf, nx, ny, p3, k1, k3, stepper):
+    lib = gf._lib.lib
+    kw = dict(nx=nx, ny=ny, Ly=2 * np.pi * ny / nx, dt=1e-4, stepper=stepper)
+    made = [lambda T: gf.TwoDNavierStokes.Problem(gf.GPU(), ν=1e-6, calcF=gf.RingForcing(5.0, 1.5, 0.1, seed=7), T=T, **kw),
+            lambda T: gf.SingleLayerQG.Problem(gf.GPU(), β=2.0, μ=0.1, U=0.2, deformation_radius=0.7, T=T,
+                                               eta=lambda x, y: 0.1 * np.cos(x), **kw)]
+    for make, T in ((made[0], np.float64), (made[1], np.float64), (made[1], np.float32)):
+        sols = []
+        for timed in (0, 1):
+            p = make(T)
+            gf.set_schedule(p, 0, 0, p3)
+            gf.set_splits(p, k1, 0, k3)
+            p.sol = state(ny, nx, T)
+            assert lib.gf_timing(p._ctx, timed) == 0
+            gf.stepforward(p, 4)
+            gf.stepforward(p, 1)
+            sols.append(p.sol)
+        assert np.isfinite(sols[0]).all() and np.array_equal(sols[0], sols[1])
+
+
+@pytest.mark.parametrize("nx,ny,p3,k1,k3", [(32, 32, 4, 1, 0), (64, 256, 4, 1, 1), (64, 1024, 8, 1, 1), (128, 2048, 8, 0, 1)])
+def test_fused_stages_match_the_oracle(gf, nx, ny, p3, k1, k3):
+    kw = dict(nx=nx, ny=ny, Ly=2 * np.pi * ny / nx, dt=1e-3, stepper="FilteredETDRK4")
+    p = gf.SingleLayerQG.Problem(gf.GPU(), β=2.0, μ=0.1, ν=1e-5, **kw)
+    gf.set_schedule(p, 0, 0, p3)
+    gf.set_splits(p, k1, 1, k3)
+    r = osl.Problem(beta=2.0, mu=0.1, nu=1e-5, **kw)
+    p.sol = state(ny, nx, np.float64)
+    r.sol[...] = p.sol
+    gf.stepforward(p, 5)
+    off.stepforward(r, 5)
+    assert rel(p.sol, r.sol) < 1e-12
