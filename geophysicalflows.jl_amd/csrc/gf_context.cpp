@@ -414,7 +414,7 @@ struct Ctx final : CtxBase {
     if (d.forcing == GF_FORCING_FIXED) Fh.alloc(sizeof(C) * fsz * nl);   // zero until gf_set_forcing
     if (nl > 1 && d.mu != 0) psib.alloc(sizeof(C) * fsz);
     Sched tuned;
-    if (tunable() && sched_lookup(sched_key(), tuned)) {
+    if (tunable() && (sched_lookup(sched_key(), tuned) || sched_by_length(sched_key(), tuned))) {
       for (int k = 0; k < 3; ++k) sched[k] = tuned.p[k];
       for (int k = 0; k < 3; ++k) split[k] = tuned.split[k];
     }
@@ -872,21 +872,30 @@ struct Ctx final : CtxBase {
   }
   // The y passes of consecutive evaluations (K3 of one stage, K1 of the next) run as one launch where
   // that kernel is built for the schedule: P and the columns per group as K3's, three groups per column
-  // where K1 has a field per workgroup row.  In the steps of such problems K1 too runs at K3's P, so
-  // that a step has the same bits whichever of its stages are fused (the first of a call, every
-  // stage while the kernels are timed one by one, and all under a split it is not built for, are not).
-  int ypass_p() const { return sched[2] ? sched[2] : sched_default(d.ny); }
-  bool ypass_fusable() const {
-    return tunable() && ystage_built(d.ny, ypass_p(), split[0] ? 3 : 1, split[2] && k3_single_column(d.ny, ypass_p()) ? 1 : 2);
+  // where K1 has a field per workgroup row and they are built, else one.  From 2048 points P is at least 8:
+  // at 4 a column is 512 threads that wait for each other at every exchange (2048^2 FP32 step 208 us at
+  // 4, 193 at 8).  In the steps of such problems K1 and K3 too run at that P, so that a step has the
+  // same bits whichever of its stages are fused (the first of a call, every stage while the kernels are
+  // timed one by one, and all under a split it is not built for, are not).
+  int ypass_p() const {
+    const int p = sched[2] ? sched[2] : sched_default(d.ny);
+    return d.ny >= 2048 && p < 8 ? 8 : p;
   }
+  int ypass_groups() const {   // thread groups per column, 0: not fused
+    if (!tunable()) return 0;
+    const int p = ypass_p(), cpw = split[2] && k3_single_column(d.ny, p) ? 1 : 2;
+    if (split[0] && ystage_built(d.ny, p, 3, cpw)) return 3;
+    return ystage_built(d.ny, p, 1, cpw) ? 1 : 0;
+  }
+  bool ypass_fusable() const { return ypass_groups() > 0; }
   // One stage of a run of stages on stream st: K1 unless the stage before has left its fields (first),
   // the x pass, then K3 (last) or K3 with the next stage's K1.
-  void stage_launch(K1Args<T>& a, const K2Args<T>& b, const K3Args<T>& c, bool first, bool last, hipStream_t st) {
-    if (tunable()) a.p = ypass_p();
+  void stage_launch(K1Args<T>& a, const K2Args<T>& b, K3Args<T>& c, bool first, bool last, hipStream_t st) {
+    if (tunable()) a.p = c.p = ypass_p();
     if (first) { rec(0, true); launch_k1<T>(d.ny, a, st); rec(0, false); }
     rec(1, true); launch_k2<T>(d.nx, b, st); rec(1, false);
     if (last) { rec(2, true); launch_k3<T>(d.ny, c, st); rec(2, false); }
-    else launch_ystage<T>(d.ny, c, a, st);
+    else launch_ystage<T>(d.ny, ypass_groups(), c, a, st);
   }
 
   // the stages of one step: (calcN input, epilogue) pairs

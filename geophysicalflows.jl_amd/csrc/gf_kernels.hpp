@@ -288,8 +288,8 @@ template <typename T> void launch_pv_from_psi(const PvArgs<T>& a, hipStream_t s)
 template <typename T> void launch_k1(int ny, const K1Args<T>& a, hipStream_t s);
 template <typename T> void launch_k2(int nx, const K2Args<T>& a, hipStream_t s);
 template <typename T> void launch_k3(int ny, const K3Args<T>& a, hipStream_t s);
-// K3 of the stage c, then K1 (args a) of the next evaluation, on the same columns
-template <typename T> void launch_ystage(int ny, const K3Args<T>& c, const K1Args<T>& a, hipStream_t s);
+// K3 of the stage c, then K1 (args a) of the next evaluation, on the same columns (groups 1 or 3)
+template <typename T> void launch_ystage(int ny, int groups, const K3Args<T>& c, const K1Args<T>& a, hipStream_t s);
 template <typename T> void launch_to_julia(const Geo<T>& g, const cplx<T>* src, cplx<T>* dst, int nl, hipStream_t s);
 template <typename T> void launch_from_julia(const Geo<T>& g, const cplx<T>* src, cplx<T>* dst, int nl, hipStream_t s);
 template <typename T> void launch_mask(const Geo<T>& g, cplx<T>* sol, int nl, hipStream_t s);
@@ -319,7 +319,7 @@ constexpr bool k3_single_column(int n, int p) { return n / p >= 64; }
 constexpr bool ystage_built(int n, int p, int ng, int cpw) {
   if (n < 32 || n > 4096 || (cpw == 1 && !k3_single_column(n, p))) return false;
   if (ng == 3) return n <= 1024 && (p == 4 || p == 8) && 3 * cpw * (n / p) <= 1024;
-  return n >= 1024 && ((p == 4 && n <= 2048) || p == 8 || (p == 16 && n == 4096));
+  return n >= 1024 && ((p == 4 && n == 1024) || p == 8 || (p == 16 && n == 4096));
 }
 // Workgroups of a launch with G column pairs per workgroup over ncols columns; with quads and
 // G = 1, a multiple of 16 (pair_of_block puts the two pairs of a block on one XCD).

@@ -1697,7 +1697,9 @@ void k2_n(const K2Args<T>& a, hipStream_t s) {
   if constexpr (NL == 1) {
     if (tuned && a.p == 4) { if constexpr (PCand<N>::has(4) && PY<N>::P != 4) { k2_np<T, N, 1, 4>(a, s); return; } }
     if (tuned && a.p == 8) { if constexpr (PCand<N>::has(8) && PY<N>::P != 8) { k2_np<T, N, 1, 8>(a, s); return; } }
-    if (tuned && a.p == 16) { if constexpr (PCand<N>::has(16) && PY<N>::P != 16) { k2_np<T, N, 1, 16>(a, s); return; } }
+    // (with background gradients a thread holds three products: 16 points of them spill, so those
+    // run at 8 where the schedule says 16)
+    if (tuned && a.p == 16 && a.mode == K2_ADVECT) { if constexpr (PCand<N>::has(16) && PY<N>::P != 16) { k2_np<T, N, 1, 16>(a, s); return; } }
   }
   (void)tuned;
   if constexpr (NL > 1) {

@@ -109,6 +109,31 @@ bool sched_lookup(const SchedKey& key, Sched& out) {
   return true;
 }
 
+bool sched_by_length(const SchedKey& key, Sched& out) {
+  std::lock_guard<std::mutex> g(mu);
+  // the best square entry of length n: 2 points for the precision, 1 for the model
+  auto best = [&](int n) {
+    const Sched* e = nullptr;
+    int score = -1;
+    for (const auto& kv : table()) {
+      const SchedKey& k = kv.first;
+      if (k[1] != 1 || k[2] != n || k[3] != n) continue;
+      const int s = 2 * (k[4] == key[4]) + (k[0] == key[0]);
+      if (s > score) { score = s; e = &kv.second; }
+    }
+    return e;
+  };
+  const Sched* col = best(key[3]);
+  const Sched* row = best(key[2]);
+  if (!col && !row) return false;
+  out = Sched{};
+  if (col) {
+    out.p[0] = col->p[0]; out.p[2] = col->p[2];
+    out.split[0] = col->split[0]; out.split[2] = col->split[2];
+  }
+  if (row) { out.p[1] = row->p[1]; out.split[1] = row->split[1]; }
+  return true;
+}
 void sched_store(const SchedKey& key, const Sched& s) {
   std::lock_guard<std::mutex> g(mu);
   table()[key] = s;

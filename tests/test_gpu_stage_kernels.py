@@ -45,7 +45,7 @@ def test_a_group_per_field_gives_the_plain_x_pass(gf, nx, ny, p2, dtype):
 # and of several waves, one group, pairs and single columns) and rectangles
 FORMS = [(32, 32, 4, 1, 0), (32, 32, 8, 1, 0), (64, 64, 4, 1, 0), (128, 64, 8, 1, 0), (64, 128, 4, 1, 0), (32, 256, 4, 1, 1),
          (256, 256, 8, 1, 0), (64, 512, 8, 1, 1), (64, 512, 4, 1, 0), (32, 1024, 4, 1, 1), (32, 1024, 8, 1, 0), (64, 1024, 8, 0, 1),
-         (32, 2048, 4, 0, 0), (64, 2048, 8, 0, 1), (32, 4096, 8, 0, 0), (32, 4096, 8, 0, 1), (32, 4096, 16, 0, 0)]
+         (32, 2048, 4, 1, 0), (64, 2048, 8, 0, 1), (32, 4096, 8, 0, 0), (32, 4096, 8, 0, 1), (32, 4096, 16, 0, 0)]
 
 
 @pytest.mark.parametrize("nx,ny,p3,k1,k3", FORMS)
