@@ -889,13 +889,14 @@ struct Ctx final : CtxBase {
   }
   bool ypass_fusable() const { return ypass_groups() > 0; }
   // One stage of a run of stages on stream st: K1 unless the stage before has left its fields (first),
-  // the x pass, then K3 (last) or K3 with the next stage's K1.
-  void stage_launch(K1Args<T>& a, const K2Args<T>& b, K3Args<T>& c, bool first, bool last, hipStream_t st) {
+  // the x pass, then K3, or with fuse the fused y pass, without its second half in the last stage.
+  void stage_launch(K1Args<T>& a, const K2Args<T>& b, K3Args<T>& c, bool fuse, bool first, bool last, hipStream_t st) {
     if (tunable()) a.p = c.p = ypass_p();
     if (first) { rec(0, true); launch_k1<T>(d.ny, a, st); rec(0, false); }
     rec(1, true); launch_k2<T>(d.nx, b, st); rec(1, false);
-    if (last) { rec(2, true); launch_k3<T>(d.ny, c, st); rec(2, false); }
-    else launch_ystage<T>(d.ny, ypass_groups(), c, a, st);
+    if (last) a.ncols = 0;
+    if (fuse) launch_ystage<T>(d.ny, ypass_groups(), c, a, st);
+    else { rec(2, true); launch_k3<T>(d.ny, c, st); rec(2, false); }
   }
 
   // the stages of one step: (calcN input, epilogue) pairs
@@ -1090,7 +1091,7 @@ struct Ctx final : CtxBase {
     for (int k = 0; k < ns; ++k) {
       make_args(ins[k], epis[k], false, a, b, c);
       c.fstep_dev = fstep_dev;
-      stage_launch(a, b, c, !fuse, !fuse, stream);
+      stage_launch(a, b, c, fuse, !fuse, !fuse, stream);
     }
     HIPCHECK(hipGetLastError());
     if (fstep_dev) launch_counter(step_dev.as<int64_t>(), 1, 1, stream);
@@ -1147,7 +1148,7 @@ struct Ctx final : CtxBase {
           }
           make_args(ins[k], epis[k], full, ka, kb, kc);
           const bool last = !fuse || (full && k == ns - 1);
-          stage_launch(ka, kb, kc, !fields, last, stream);
+          stage_launch(ka, kb, kc, fuse, !fields, last, stream);
           fields = !last;
         }
         HIPCHECK(hipGetLastError());
@@ -1173,8 +1174,18 @@ struct Ctx final : CtxBase {
   }
   void get_state(void* dst, hipMemcpyKind kind) override {
     const size_t bytes = sizeof(C) * (size_t)g.nkr * d.ny * nl;
-    launch_to_julia<T>(g, sol.as<C>(), jl.as<C>(), nl, stream);
-    HIPCHECK(hipMemcpyAsync(dst, jl.p, bytes, kind == hipMemcpyDeviceToHost ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, stream));
+    // into memory of this device the conversion writes straight (2048^2 FP64: 16 us instead of 16 + 12,
+    // and one queued operation fewer at every size); what it cannot store to goes by way of jl
+    hipPointerAttribute_t at{};
+    if (kind == hipMemcpyDeviceToDevice && (uintptr_t)dst % sizeof(C) == 0 && hipPointerGetAttributes(&at, dst) == hipSuccess &&
+        at.type == hipMemoryTypeDevice && at.device == device) {
+      launch_to_julia<T>(g, sol.as<C>(), (C*)dst, nl, stream);
+      HIPCHECK(hipGetLastError());
+    } else {
+      if (kind == hipMemcpyDeviceToDevice) (void)hipGetLastError();   // (a pointer the runtime does not know)
+      launch_to_julia<T>(g, sol.as<C>(), jl.as<C>(), nl, stream);
+      HIPCHECK(hipMemcpyAsync(dst, jl.p, bytes, kind == hipMemcpyDeviceToHost ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, stream));
+    }
     HIPCHECK(hipStreamSynchronize(stream));
   }
   void set_physical(const void* f) override {
@@ -1550,7 +1561,7 @@ struct Ctx final : CtxBase {
         make_args(q == 0 ? s0 : ins[q], epis[q], false, a, b, k);
         k.sol = s0; k.s1 = b1; k.s2 = b2; k.nsave = slot(i, q + 1, tp);
         if (q == 3) { k.sol_out = slot(i + 1, 0, tp); k.nonfinite = nullptr; }
-        stage_launch(a, b, k, !fuse || (i == 0 && q == 0), !fuse || (i == n - 1 && q == 3), st);
+        stage_launch(a, b, k, fuse, !fuse || (i == 0 && q == 0), !fuse || (i == n - 1 && q == 3), st);
       }
     }
     tm.on = was;

@@ -288,7 +288,8 @@ template <typename T> void launch_pv_from_psi(const PvArgs<T>& a, hipStream_t s)
 template <typename T> void launch_k1(int ny, const K1Args<T>& a, hipStream_t s);
 template <typename T> void launch_k2(int nx, const K2Args<T>& a, hipStream_t s);
 template <typename T> void launch_k3(int ny, const K3Args<T>& a, hipStream_t s);
-// K3 of the stage c, then K1 (args a) of the next evaluation, on the same columns (groups 1 or 3)
+// K3 of the stage c, then K1 (args a) of the next evaluation, on the same columns (groups 1 or 3);
+// a.ncols = 0: the stage alone
 template <typename T> void launch_ystage(int ny, int groups, const K3Args<T>& c, const K1Args<T>& a, hipStream_t s);
 template <typename T> void launch_to_julia(const Geo<T>& g, const cplx<T>* src, cplx<T>* dst, int nl, hipStream_t s);
 template <typename T> void launch_from_julia(const Geo<T>& g, const cplx<T>* src, cplx<T>* dst, int nl, hipStream_t s);

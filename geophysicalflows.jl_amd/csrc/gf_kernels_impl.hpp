@@ -193,21 +193,12 @@ __device__ __forceinline__ cplx<T> slqg_psi(int eb, T ell2inv, cplx<T> sv, int k
   }
   return rmul(-inv_k2(kr, l, kv, lv), sv);
 }
-// Spectrum of the velocity (or psi) field `code` of a point's state sv: TwoDNS from iK = 1/|k|^2, the
-// QG models from psih = p
-template <typename T, int MODEL>
-__device__ __forceinline__ cplx<T> k1_field(int code, cplx<T> sv, T iK, cplx<T> p, T kv, T lv) {
-  if constexpr (MODEL == M_TWODNS) {
-    // uh = i l invK sol, vh = -i kr invK sol (src/twodnavierstokes.jl:254-255)
-    if (code == F_U) { const T aa = lv * iK; return mk(-aa * sv.im, aa * sv.re); }
-    if (code == F_V) { const T bb = kv * iK; return mk(bb * sv.im, -bb * sv.re); }
-    return rmul(-iK, sv);
-  } else {
-    // uh = -i l psih, vh = i kr psih (src/singlelayerqg.jl:360-361)
-    if (code == F_U) return mk(lv * p.im, -lv * p.re);
-    if (code == F_V) return mk(-kv * p.im, kv * p.re);
-    return p;
-  }
+// Spectrum of the velocity (or psi) field `code` of a point's psih = p: uh = -i l psih, vh = i kr psih
+// (src/singlelayerqg.jl:360-361; TwoDNS with psih = -invKrsq sol, src/twodnavierstokes.jl:254-255)
+template <typename T> __device__ __forceinline__ cplx<T> k1_field(int code, cplx<T> p, T kv, T lv) {
+  if (code == F_U) return mk(lv * p.im, -lv * p.re);
+  if (code == F_V) return mk(-kv * p.im, kv * p.re);
+  return p;
 }
 
 // Body of K1 for block blk of column pairs; lds holds 2G padded N-point buffers and
@@ -301,7 +292,7 @@ __device__ __forceinline__ void k1_body(const K1Args<T>& a, int blk, cplx<T>* __
         const T lv = lwave(g, l);
         cplx<T> r;
         if (code == F_RAW || code == F_Q) r = svs[q];
-        else r = k1_field<T, MODEL>(code, svs[q], MODEL == M_TWODNS ? iK[q] : (T)0, ps[q], kv, lv);
+        else r = k1_field(code, MODEL == M_TWODNS ? rmul(-iK[q], svs[q]) : ps[q], kv, lv);
         // normalised inverse = conj(F(conj(x)))/(nx ny); the scale is a power of two
         w[0][q] = mk(r.re * nrm, -(r.im * nrm));
       }

@@ -4,9 +4,9 @@
 // modes, K1 reads those modes back, forms u, v and q and transforms them inversely.  Inside a
 // run of stages one kernel does both, so a stage is two launches (x pass, y pass) instead of
 // three, the new state is not read back, and the intermediate states of ETDRK4 that only the
-// next K1 reads (stages 2 and 3) are not written at all.  The first stage of a call starts with K1
-// and the last one ends with K3; every expression is the one those kernels evaluate
-// (stage_point, k1_field), so the results are theirs bit for bit.
+// next K1 reads (stages 2 and 3) are not written at all.  The first stage of a call starts with K1;
+// the last one's launch leaves the fields out (K1's ncols = 0).  Every expression is the one K3 and K1
+// evaluate (stage_point, k1_field), so the results are theirs bit for bit.
 //
 // NG = 3: three thread groups per column (or column pairs).  Groups 0 and 1 transform the two fluxes
 // side by side, the modes of the column are stepped by all three, and each transforms one of u, v, q:
@@ -27,14 +27,18 @@ template <int N, int P, int NG, int CPW> struct YS {
   static constexpr int GT = CPW * G * TPT;             // threads per group, whole waves
   static constexpr int X = GT == 64 ? X_WAVE : X_LDS;
   static constexpr int QN = (P + NG - 1) / NG;         // modes a thread steps
+  // single 4096-point columns of 512 threads: two of them fit a CU's LDS, so 4 waves per SIMD are
+  // wanted (128 VGPRs, some spilled: 4096^2 RK4 stages 248 -> 212 us)
+  static constexpr bool TIGHT = NG == 1 && CPW == 1 && TPT == 512;
 };
 template <typename T, int NY, int P, int NG, int CPW, int MODEL, int EPI>
-__global__ __launch_bounds__((NG * YS<NY, P, NG, CPW>::GT)) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__((NG * YS<NY, P, NG, CPW>::GT)) __attribute__((amdgpu_waves_per_eu((YS<NY, P, NG, CPW>::TIGHT ? 4 : 2))))
 void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
   using Y = YS<NY, P, NG, CPW>;
   constexpr int TPT = Y::TPT, G = Y::G, GT = Y::GT, X = Y::X, PG = XPad<T>::G;
   constexpr int BUF = CPW == 2 ? G * PairLds<T, NY>::value : LdsN<NY>::value;
   constexpr bool FR = NG == 1 && sizeof(T) == 8 && NY >= 2048;
+  constexpr bool TIGHT = Y::TIGHT;
   __shared__ cplx<T> lds[NG * BUF];
   __shared__ cplx<T> tw[TwPlan<NY, P>::size()];
   const Geo<T>& g = c.g;
@@ -141,25 +145,24 @@ void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
   const unsigned long long badm = __ballot(bad);
   if (badm != 0 && c.nonfinite != nullptr && (int)(threadIdx.x & 63) == __ffsll(badm) - 1) *c.nonfinite = 1;
 
-  // the next calcN!'s fields of the kept columns
+  // the next calcN!'s fields of the kept columns (none after the last stage of a call)
+  if (a.ncols == 0) return;
   const bool out = active && kr < a.ncols;
   if (CPW == 1 && kr >= a.ncols) return;               // (a single column is its whole workgroup's)
-  T iK[P];
   cplx<T> ps[P];
 #pragma unroll
   for (int q = 0; q < P; ++q) {
     const int l = t + TPT * q;
-    iK[q] = MODEL == M_TWODNS ? inv_k2(kr, l, kv, lwave(g, l)) : (T)0;
-    ps[q] = MODEL == M_TWODNS ? czero<T>() : slqg_psi(a.eb, a.ell2inv, sv[q], kr, l, kv, lwave(g, l));
+    ps[q] = MODEL == M_TWODNS ? rmul(-inv_k2(kr, l, kv, lwave(g, l)), sv[q]) : slqg_psi(a.eb, a.ell2inv, sv[q], kr, l, kv, lwave(g, l));
   }
   const T nrm = g.inv_norm;
 #pragma unroll
   for (int f = 0; f < (NG == 1 ? 3 : 1); ++f) {
-    const int field = NG == 1 ? f : grp;               // u, v, q (Fields<MODEL, FS_CALCN>)
+    // u, v, q (Fields<MODEL, FS_CALCN>); q first where registers are short: after it only psi is held
+    const int field = NG > 1 ? grp : (TIGHT ? 2 - f : f);
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-      const T lv = lwave(g, t + TPT * q);
-      const cplx<T> r = field == 2 ? sv[q] : k1_field<T, MODEL>(field == 0 ? F_U : F_V, sv[q], iK[q], ps[q], kv, lv);
+      const cplx<T> r = field == 2 ? sv[q] : k1_field(field == 0 ? F_U : F_V, ps[q], kv, lwave(g, t + TPT * q));
       w[0][q] = mk(r.re * nrm, -(r.im * nrm));
     }
     fft_forward<T, NY, P, 1, FR, X>(w, L, t, tw);
@@ -178,16 +181,23 @@ void ystage_go(const K3Args<T>& c, const K1Args<T>& a, hipStream_t s) {
   if (c.ncols <= 0) return;
   const dim3 grid(nblk), blk(NG * Y::GT);
   if constexpr (NG == 1 && N >= 2048) {
-    // one kernel per ETDRK4 stage, as K3 has them: the stage's registers set the occupancy
+    // one kernel per stage: its registers set the occupancy
     switch (c.epi) {
+      case E_FE: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_FE>), grid, blk, 0, s, c, a); return;
+      case E_AB3: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_AB3>), grid, blk, 0, s, c, a); return;
+      case E_RK1: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_RK1>), grid, blk, 0, s, c, a); return;
+      case E_RK2: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_RK2>), grid, blk, 0, s, c, a); return;
+      case E_RK3: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_RK3>), grid, blk, 0, s, c, a); return;
+      case E_RK4: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_RK4>), grid, blk, 0, s, c, a); return;
       case E_ETD1: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_ETD1>), grid, blk, 0, s, c, a); return;
       case E_ETD2: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_ETD2>), grid, blk, 0, s, c, a); return;
       case E_ETD3: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_ETD3>), grid, blk, 0, s, c, a); return;
       case E_ETD4: GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, E_ETD4>), grid, blk, 0, s, c, a); return;
-      default: break;
+      default: return;
     }
+  } else {
+    GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, -1>), grid, blk, 0, s, c, a);
   }
-  GF_LAUNCH((ystage_kernel<T, N, P, NG, CPW, MODEL, -1>), grid, blk, 0, s, c, a);
 }
 template <typename T, int N, int P, int NG>
 void ystage_p(const K3Args<T>& c, const K1Args<T>& a, hipStream_t s) {
