@@ -1768,6 +1768,11 @@ struct BatchCtx final : CtxBase {
   DevBuf items[4][2];
   DevBuf work[3][2];
   int nwork[3][2] = {};
+  DevBuf work2[2][2];      // the two-launch form: x pass, y pass
+  int nwork2[2][2] = {};
+  int nmax = 0;            // largest member
+  int groups = 3;          // its thread groups per entry
+  bool two_launch = true;  // no member's stage reads a state that the fused y pass does not store
   KernelTimer tm;
   bool ring = false;       // some member has stochastic ring forcing
   bool ab3m = false;       // the members step with AB3 / FilteredAB3
@@ -1808,6 +1813,18 @@ struct BatchCtx final : CtxBase {
     if (ring) ctr.alloc(sizeof(int64_t));
     std::vector<BatchItem<T>> h(n);
     k2_plain = true;
+    two_launch = true;
+    nmax = inst[ord[0]]->d.nx;
+    long entries = 0;
+    for (auto& m : inst) {
+      two_launch = two_launch && m->d.model != GF_MODEL_MLQG;
+      entries += batch2_blocks(0, m->d.nx, m->d.ny, 3);
+    }
+    // Three groups per entry while the x pass has at most 10 workgroups per CU of them, else one. FP64
+    // SingleLayerQG FilteredRK4, us per step for 3 groups / 1 group (three launches before): 8 x 256^2, 4 per
+    // CU, 110 / 129 (170); 32 x 64^2 + 24 x 128^2 + 8 x 256^2, 8 per CU, 149 / 161 (196); twice that, 16 per CU,
+    // 242 / 197 (240); 512 x 64^2, 16 per CU, 218 / 173 (210); 8 times that, 64 per CU, 893 / 597 (659).
+    groups = entries <= 10 * 256 ? 3 : 1;
     for (int full = 0; full < 2; ++full) {
       for (int k = 0; k < nst; ++k) {
         for (int i = 0; i < n; ++i) {
@@ -1840,13 +1857,35 @@ struct BatchCtx final : CtxBase {
         work[kc][full].alloc(sizeof(BatchWork) * w.size());
         HIPCHECK(dw::copy(work[kc][full].p, w.data(), sizeof(BatchWork) * w.size(), hipMemcpyHostToDevice));
       }
+      for (int y = 0; y < 2; ++y) {
+        std::vector<BatchWork> w;
+        for (int i : ord) {
+          const Ctx<T>& m = *inst[i];
+          const int nb = batch2_blocks(y, m.d.nx, y == 0 ? m.d.ny : (full || ab3m ? m.g.nkr : m.g.kmax), groups);
+          for (int b = 0; b < nb; ++b) w.push_back(BatchWork{i, b});
+        }
+        nwork2[y][full] = (int)w.size();
+        work2[y][full].alloc(sizeof(BatchWork) * w.size());
+        if (!w.empty()) HIPCHECK(dw::copy(work2[y][full].p, w.data(), sizeof(BatchWork) * w.size(), hipMemcpyHostToDevice));
+      }
     }
   }
 
-  void step_launches(int full) {
+  // the kernel classes one by one: while they are timed, in the persistent form, and where the two-launch
+  // form does not serve a member
+  bool fused() const { return two_launch && !tm.on && !persistent; }
+  // one step; first: the members' fields are not there yet, last: no stage follows it
+  void step_launches(int full, bool first, bool last) {
     tm.mark(stream);
     for (int k = 0; k < nst; ++k) {
       const BatchItem<T>* it = items[k][full].as<BatchItem<T>>();
+      if (fused()) {
+        const BatchWork *wx = work2[0][full].as<BatchWork>(), *wy = work2[1][full].as<BatchWork>();
+        if (first && k == 0) launch_batch_y<T>(it, wy, nwork2[1][full], nmax, groups, 0, stream);
+        launch_batch_x<T>(it, wx, nwork2[0][full], nmax, groups, k2_plain, stream);
+        launch_batch_y<T>(it, wy, nwork2[1][full], nmax, groups, last && k == nst - 1 ? 2 : 1, stream);
+        continue;
+      }
       if (persistent) {
         const BatchStageWork sw{{work[0][full].as<BatchWork>(), work[1][full].as<BatchWork>(), work[2][full].as<BatchWork>()},
                                 {nwork[0][full], nwork[1][full], nwork[2][full]}};
@@ -1875,7 +1914,7 @@ struct BatchCtx final : CtxBase {
   bool persistent = false;
   void set_persistent(int enable) override { persistent = enable != 0; }
   void build_graph() {
-    gexec = dw::capture(stream, [&] { step_launches(0); });
+    gexec = dw::capture(stream, [&] { step_launches(0, false, false); });
   }
 
   void step(int n) override {
@@ -1905,11 +1944,12 @@ struct BatchCtx final : CtxBase {
           m->prevsol_valid = true;
         }
       }
-      if (!last && v == 0 && graphs && !tm.on && !persistent) {
+      // (the first step of a call in the two-launch form starts with K1: the captured one does not)
+      if (!last && v == 0 && graphs && !tm.on && !persistent && !(s == 0 && fused())) {
         if (!gexec) build_graph();
         HIPCHECK(hipGraphLaunch(gexec, stream));
       } else {
-        step_launches(v);
+        step_launches(v, s == 0, last);
       }
       for (auto& m : inst) { m->t += m->d.dt; m->stepno += 1; }
     }

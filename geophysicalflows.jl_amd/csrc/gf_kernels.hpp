@@ -358,6 +358,13 @@ struct BatchWork {
 // plain (K = 2): every member's x pass is K2_ADVECT, which selects the kernel without the
 // background-gradient body
 template <typename T, int K> void launch_batch(const BatchItem<T>* items, const BatchWork* work, int nwork, int plain, hipStream_t s);
+// The two-launch form (gf_batch_y_impl.hpp): the x pass and the fused y pass of one stage for every
+// instance; nmax: the largest instance; groups: thread groups per entry (1 or 3); mode 0: K1 alone, 1: K3 and
+// the next stage's K1, 2: K3 alone.
+template <typename T> void launch_batch_x(const BatchItem<T>* items, const BatchWork* work, int nwork, int nmax, int groups, int plain, hipStream_t s);
+template <typename T> void launch_batch_y(const BatchItem<T>* items, const BatchWork* work, int nwork, int nmax, int groups, int mode, hipStream_t s);
+// workgroups of that form's x pass (y = 0, count = ny) or y pass (y = 1, count = columns)
+int batch2_blocks(int y, int n, int count, int groups);
 // The three work tables of one stage (K1, K2, K3 entries) for the persistent stage launch.
 struct BatchStageWork {
   const BatchWork* w[3];

@@ -357,8 +357,9 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
   return (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
 }
 
-// Body of K2 for block blk of row pairs; lds holds G padded N-point buffers.
-template <typename T, int NX, int P, int G, int MODE, int NL>
+// Body of K2 for block blk of row pairs; lds holds G padded N-point buffers.  X: the barriers of its
+// exchanges (X_WAVE where the workgroup is one wave).
+template <typename T, int NX, int P, int G, int MODE, int NL, int X = X_FULL>
 __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __restrict__ lds,
                                         const cplx<T>* __restrict__ tw) {
   constexpr int TPT = NX / P;
@@ -385,10 +386,10 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
         }
         w[0][q] = mk(r0, r1);
       }
-      fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2)>(w, L, t, tw);
+      fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2), X>(w, L, t, tw);
 #pragma unroll
       for (int q = 0; q < P; ++q) L[padg<XPad<T>::G>(t) + padg<XPad<T>::G>(TPT * q)] = w[0][q];
-      __syncthreads();
+      xbarrier<X>();
       if (active) {
         cplx<T>* o = a.out + f * a.ostride;
         for (int it = t; it < 2 * a.kout; it += TPT) {
@@ -396,7 +397,7 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
           o[boff(kr, y0 + row, ny)] = split_row(L[padg<XPad<T>::G>(kr)], L[padg<XPad<T>::G>((NX - kr) & (NX - 1))], row);
         }
       }
-      __syncthreads();
+      xbarrier<X>();
     }
   } else if constexpr (MODE == K2_INVERSE_OUT) {
     // nfields mixed fields -> physical rows; fields paired (f, f+1) per row
@@ -413,7 +414,7 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
           const cplx<T> B = two ? herm_load<T, NX>(fb, k, y0 + row, ny, a.kin, active) : czero<T>();
           w[0][q] = mk(A.re - B.im, -(A.im + B.re));     // conj(A + i B)
         }
-        fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2)>(w, L, t, tw);
+        fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2), X>(w, L, t, tw);
         if (active) {
 #pragma unroll
           for (int q = 0; q < P; ++q) {
@@ -458,7 +459,7 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
         w[0][q] = mk(A[q].re - B[q].im, -(A[q].im + B[q].re));     // conj(A + i B)
         if (k > 0 && k < NX / 2) L[padg<XPad<T>::G>(NX - k)] = mk(A[q].re + B[q].im, A[q].im - B[q].re);
       }
-      __syncthreads();
+      xbarrier<X>();
 #pragma unroll
       for (int q = 0; q < P; ++q) {
         if (TPT * q + TPT - 1 <= NX / 2) continue;      // every lane of this q holds k <= NX/2
@@ -466,18 +467,18 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
         if (k <= NX / 2) continue;
         w[0][q] = L[padg<XPad<T>::G>(k)];
       }
-      __syncthreads();
+      xbarrier<X>();
     };
     auto inverse_rows = [&](const cplx<T>* f, cplx<T> (&w)[1][P]) {
       load_rows(f, w);
-      fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2)>(w, L, t, tw);             // row y0 = Re, row y0 + 1 = -Im
+      fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2), X>(w, L, t, tw);             // row y0 = Re, row y0 + 1 = -Im
     };
     auto forward_rows = [&](cplx<T>* o, cplx<T> (&w)[1][P]) {
-      fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2)>(w, L, t, tw);             // of (row y0 + i row y0 + 1)
+      fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2), X>(w, L, t, tw);             // of (row y0 + i row y0 + 1)
       const MirrorSlots<NX, TPT, XPad<T>::G> ms(t);
 #pragma unroll
       for (int q = 0; q < P; ++q) L[ms.k(q)] = w[0][q];
-      __syncthreads();
+      xbarrier<X>();
       if (active) {
 #pragma unroll
         for (int i = 0; i < MAXI; ++i) {
@@ -489,7 +490,7 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
           }
         }
       }
-      __syncthreads();
+      xbarrier<X>();
     };
     T q0[P], q1[P];
     {
@@ -549,7 +550,7 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
           const cplx<T> B = herm_load<T, NX>(fb, k, yb, ny, a.kin, active);
           wr[0][q] = mk(A.re - B.im, -(A.im + B.re));     // conj(A + i B)
         }
-        fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2)>(wr, L, t, tw);
+        fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2), X>(wr, L, t, tw);
 #pragma unroll
         for (int q = 0; q < P; ++q) w[r][q] = wr[0][q];
       }
@@ -601,7 +602,7 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
         cplx<T> zr[1][P];
 #pragma unroll
         for (int q = 0; q < P; ++q) zr[0][q] = z[r][q];
-        fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2)>(zr, L, t, tw);
+        fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2), X>(zr, L, t, tw);
 #pragma unroll
         for (int q = 0; q < P; ++q) z[r][q] = zr[0][q];
       }
@@ -612,7 +613,7 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
       for (int row = 0; row < 2; ++row) {
 #pragma unroll
         for (int q = 0; q < P; ++q) L[ms.k(q)] = z[row][q];
-        __syncthreads();
+        xbarrier<X>();
         cplx<T> Arow[MAXI], Brow[MAXI];
 #pragma unroll
         for (int i = 0; i < MAXI; ++i) {
@@ -623,12 +624,12 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
             Brow[i] = split_row(Wk, Wm, 1);
           }
         }
-        __syncthreads();
+        xbarrier<X>();
         if constexpr (FULL) {
           // this row's C = u Qx + v Qy spectrum from the packed (C0 + i C1) transform
 #pragma unroll
           for (int q = 0; q < P; ++q) L[ms.k(q)] = z[2][q];
-          __syncthreads();
+          xbarrier<X>();
 #pragma unroll
           for (int i = 0; i < MAXI; ++i) {
             const int kr = t + i * TPT;
@@ -639,7 +640,7 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
               Arow[i] = mk(kv * Arow[i].im - Cv.re, -kv * Arow[i].re - Cv.im);
             }
           }
-          __syncthreads();
+          xbarrier<X>();
         }
         if (active) {
 #pragma unroll
@@ -845,7 +846,7 @@ void k2_kernel(const K2Args<T> a) {
   __shared__ cplx<T> tw[TwPlan<NX, P>::size()];
   load_twiddles<T, NX, P>(tw, a.tw);
   __syncthreads();
-  k2_body<T, NX, P, G, MODE, NL>(a, xcd_block(blockIdx.x, gridDim.x), lds, tw);
+  k2_body<T, NX, P, G, MODE, NL, (G * (NX / P) == 64 ? X_WAVE : X_FULL)>(a, xcd_block(blockIdx.x, gridDim.x), lds, tw);
 }
 
 // ---------------------------------------------------------------------------
@@ -869,20 +870,16 @@ template <int NX, int P> struct K2P {
   static constexpr bool fits(int size) { return 3 * GT <= 1024 && 3 * G * LdsN<NX>::value * size <= 120 * 1024; }
 };
 template <typename T, int NX, int P, bool FULL>
-__global__ __launch_bounds__((3 * K2P<NX, P>::GT)) __attribute__((amdgpu_waves_per_eu(2)))
-void k2_group_kernel(const K2Args<T> a) {
+__device__ __forceinline__ void k2_group_body(const K2Args<T>& a, int blk, int jl, cplx<T>* __restrict__ lds, cplx<T>* __restrict__ tw) {
   using K = K2P<NX, P>;
   constexpr int TPT = K::TPT, G = K::G, X = K::X, PG = XPad<T>::G;
   constexpr int MAXI = (NX / 2 + 1 + TPT - 1) / TPT;
   constexpr int QH = P / 2 + 1;                        // the q with TPT q <= NX/2
-  __shared__ cplx<T> lds[3 * G * LdsN<NX>::value];
-  __shared__ cplx<T> tw[TwPlan<NX, P>::size()];
   const Geo<T>& g = a.g;
   const int ny = g.ny;
   const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x / K::GT);
   const int t = (int)threadIdx.x % TPT, slot = ((int)threadIdx.x % K::GT) / TPT;
-  const int jl = (int)blockIdx.y;
-  const int rp = xcd_block(blockIdx.x, gridDim.x) * G + slot;
+  const int rp = blk * G + slot;
   const bool active = rp < ny / 2;
   const int y0 = 2 * rp;
   auto buffer = [&](int f) { return lds + (f * G + slot) * LdsN<NX>::value; };
@@ -1022,6 +1019,14 @@ void k2_group_kernel(const K2Args<T> a) {
       at(o, boff32(kr, y0 + 1, ny)) = r1[i];
     }
   }
+}
+
+template <typename T, int NX, int P, bool FULL>
+__global__ __launch_bounds__((3 * K2P<NX, P>::GT)) __attribute__((amdgpu_waves_per_eu(2)))
+void k2_group_kernel(const K2Args<T> a) {
+  __shared__ cplx<T> lds[3 * K2P<NX, P>::G * LdsN<NX>::value];
+  __shared__ cplx<T> tw[TwPlan<NX, P>::size()];
+  k2_group_body<T, NX, P, FULL>(a, xcd_block(blockIdx.x, gridDim.x), (int)blockIdx.y, lds, tw);
 }
 
 // ---------------------------------------------------------------------------

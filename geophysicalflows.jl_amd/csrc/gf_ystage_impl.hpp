@@ -31,16 +31,23 @@ template <int N, int P, int NG, int CPW> struct YS {
   // wanted (128 VGPRs, some spilled: 4096^2 RK4 stages 248 -> 212 us)
   static constexpr bool TIGHT = NG == 1 && CPW == 1 && TPT == 512;
 };
-template <typename T, int NY, int P, int NG, int CPW, int MODEL, int EPI>
-__global__ __launch_bounds__((NG * YS<NY, P, NG, CPW>::GT)) __attribute__((amdgpu_waves_per_eu((YS<NY, P, NG, CPW>::TIGHT ? 4 : 2))))
-void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
+// Which halves of the fused pass a launch runs: K1 alone (the first stage of a run), both, K3 alone (the
+// last).
+enum YMode { Y_FIELDS = 0, Y_BOTH = 1, Y_STAGE = 2 };
+
+// LDS of one workgroup, in complex slots (beside the twiddle table).
+template <typename T, int N, int P, int NG, int CPW> struct YLds {
+  static constexpr int BUF = CPW == 2 ? YS<N, P, NG, CPW>::G * PairLds<T, N>::value : LdsN<N>::value;
+  static constexpr int value = NG * BUF;
+};
+
+template <typename T, int NY, int P, int NG, int CPW, int MODEL, int EPI, bool AHEAD>
+__device__ __forceinline__ void ystage_body(const K3Args<T>& c, const K1Args<T>& a, int blk, int mode, cplx<T>* __restrict__ lds,
+                                            cplx<T>* __restrict__ tw) {
   using Y = YS<NY, P, NG, CPW>;
-  constexpr int TPT = Y::TPT, G = Y::G, GT = Y::GT, X = Y::X, PG = XPad<T>::G;
-  constexpr int BUF = CPW == 2 ? G * PairLds<T, NY>::value : LdsN<NY>::value;
+  constexpr int TPT = Y::TPT, G = Y::G, GT = Y::GT, X = Y::X, PG = XPad<T>::G, BUF = YLds<T, NY, P, NG, CPW>::BUF;
   constexpr bool FR = NG == 1 && sizeof(T) == 8 && NY >= 2048;
   constexpr bool TIGHT = Y::TIGHT;
-  __shared__ cplx<T> lds[NG * BUF];
-  __shared__ cplx<T> tw[TwPlan<NY, P>::size()];
   const Geo<T>& g = c.g;
   const int grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / GT);
   const int tid = (int)threadIdx.x % GT;
@@ -48,20 +55,33 @@ void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
   if constexpr (CPW == 2) {
     const YMap<TPT> m(tid);
     t = m.t;
-    kr = 2 * (G == 1 ? pair_of_block(blockIdx.x) : (int)blockIdx.x * G + m.slot) + m.c;
+    kr = 2 * (G == 1 ? pair_of_block(blk) : blk * G + m.slot) + m.c;
     col = (int)(col_buffer<T, NY>(lds, m.slot, m.c) - lds);
   } else {
     t = tid;
-    kr = single_column(blockIdx.x);
+    kr = single_column(blk);
     col = 0;
   }
   cplx<T>* L = lds + grp * BUF + col;
-  const bool active = kr < c.ncols && kr < g.nkr;
   const T kv = krwave(g, kr);
+  cplx<T> w[1][P], sv[P];
+  if (mode == Y_FIELDS) {
+    // the state itself, masked
+    load_twiddles<T, NY, P>(tw, c.tw);
+    const bool in = kr < a.ncols && kr < g.kmax;
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const int l = t + TPT * q;
+      const cplx<T> v = at(a.sol, boff32(in ? kr : 0, l, NY));
+      sv[q] = in && kept_l(g, l) ? v : czero<T>();
+    }
+    lds_barrier();
+  } else {
+  const bool active = kr < c.ncols && kr < g.nkr;
   const int epi = EPI >= 0 ? EPI : c.epi;
 
   // the fluxes of this column: group 0 (u q)^, group 1 (v q)^
-  cplx<T> w[1][P], w1[1][NG == 1 ? P : 1];
+  cplx<T> w1[1][NG == 1 ? P : 1];
   const int krl = active ? kr : 0;
   {
     const cplx<T>* f = c.in + (long)(grp == 1 ? c.fstride : 0);
@@ -77,8 +97,8 @@ void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
   // modes per thread; with one group the registers do not hold them)
   auto row = [&](int i) { return t + TPT * (NG == 1 ? i : grp + NG * i); };
   auto mine = [&](int i) { return NG == 1 || grp + NG * i < P; };
-  StageIn<T> in[NG == 1 ? 1 : Y::QN];
-  if constexpr (NG > 1) {
+  StageIn<T> in[AHEAD ? Y::QN : 1];
+  if constexpr (AHEAD) {
 #pragma unroll
     for (int i = 0; i < Y::QN; ++i)
       in[i] = stage_load<T>(c, epi, StagePoint<T>(c, krl, mine(i) ? row(i) : t, NY, 0u));
@@ -102,7 +122,6 @@ void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
   if constexpr (NG == 1) fft_forward<T, NY, P, 1, FR, X>(w1, L, t, tw);
 
   bool bad = false;
-  cplx<T> sv[P];
   if constexpr (NG == 1) {
 #pragma unroll
     for (int q = 0; q < P; ++q) {
@@ -133,8 +152,11 @@ void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
       const int l = row(i), s = padg<PG>(l);
       const bool kept = kept_l(g, l) && kr < g.kmax;
       cplx<T> r = czero<T>();
-      if (active && (kept || c.full))
-        r = stage_point<T, 1, false, true>(c, epi, StagePoint<T>(c, kr, l, NY, 0u), in[i], kept, 0, kv, lwave(g, l), A[s], B[s], czero<T>(), c.noise, bad);
+      if (active && (kept || c.full)) {
+        const StagePoint<T> pt(c, kr, l, NY, 0u);
+        const StageIn<T> one = AHEAD ? in[AHEAD ? i : 0] : stage_load<T>(c, epi, pt);
+        r = stage_point<T, 1, false, true>(c, epi, pt, one, kept, 0, kv, lwave(g, l), A[s], B[s], czero<T>(), c.noise, bad);
+      }
       S[s] = r;
     }
     lds_barrier();
@@ -145,9 +167,11 @@ void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
   const unsigned long long badm = __ballot(bad);
   if (badm != 0 && c.nonfinite != nullptr && (int)(threadIdx.x & 63) == __ffsll(badm) - 1) *c.nonfinite = 1;
 
-  // the next calcN!'s fields of the kept columns (none after the last stage of a call)
-  if (a.ncols == 0) return;
-  const bool out = active && kr < a.ncols;
+  if (mode == Y_STAGE) return;
+  }
+
+  // the next calcN!'s fields of the kept columns
+  const bool out = kr < a.ncols && kr < g.nkr;
   if (CPW == 1 && kr >= a.ncols) return;               // (a single column is its whole workgroup's)
   cplx<T> ps[P];
 #pragma unroll
@@ -172,6 +196,14 @@ void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
       for (int q = 0; q < P; ++q) at(o, boff32(kr, t + TPT * q, NY)) = conj(w[0][q]);
     }
   }
+}
+
+template <typename T, int NY, int P, int NG, int CPW, int MODEL, int EPI>
+__global__ __launch_bounds__((NG * YS<NY, P, NG, CPW>::GT)) __attribute__((amdgpu_waves_per_eu((YS<NY, P, NG, CPW>::TIGHT ? 4 : 2))))
+void ystage_kernel(const K3Args<T> c, const K1Args<T> a) {
+  __shared__ cplx<T> lds[YLds<T, NY, P, NG, CPW>::value];
+  __shared__ cplx<T> tw[TwPlan<NY, P>::size()];
+  ystage_body<T, NY, P, NG, CPW, MODEL, EPI, (NG > 1)>(c, a, blockIdx.x, a.ncols == 0 ? Y_STAGE : Y_BOTH, lds, tw);
 }
 
 template <typename T, int N, int P, int NG, int CPW, int MODEL>

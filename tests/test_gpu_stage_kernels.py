@@ -82,3 +82,34 @@ def test_fused_stages_match_the_oracle(gf, nx, ny, p3, k1, k3):
     gf.stepforward(p, 5)
     off.stepforward(r, 5)
     assert rel(p.sol, r.sol) < 1e-12
+
+
+@pytest.mark.parametrize("counts,stepper,dtype", [((1, 1, 1, 1, 1), "ETDRK4", np.float64), ((2, 1, 1, 1, 1), "FilteredRK4", np.float32),
+                                                  ((60, 60, 60, 60, 0), "RK4", np.float64), ((700, 0, 0, 20, 8), "AB3", np.float64)])
+def test_both_ensemble_forms_match_members_stepped_alone(gf, counts, stepper, dtype):
+    # few entries run with three thread groups each, many with one; every size, the last step of a
+    # call in full; to the rounding of a few steps (a member alone has another radix schedule)
+    tol = 1e-13 if dtype == np.float64 else 2e-5
+    sizes = [n for n, c in zip((32, 64, 128, 256, 512), counts) for _ in range(c)]
+    made = []
+    for i, n in enumerate(sizes):
+        kw = dict(nx=n, dt=1e-3, stepper=stepper, μ=0.1, T=dtype)
+        if i % 2:
+            made.append((gf.TwoDNavierStokes.Problem, dict(ν=1e-5, calcF=gf.RingForcing(5.0, 1.5, 0.1, seed=i), **kw)))
+        else:
+            made.append((gf.SingleLayerQG.Problem, dict(β=2.0, U=0.2 * np.cos(2 * np.pi * np.arange(n) / n) if i % 4 else 0.1, **kw)))
+    ens = gf.Ensemble(made)
+    look = sorted({0, 1, 2, 3, len(sizes) - 1, len(sizes) - 2} | {sizes.index(n) for n in set(sizes)})
+    starts = {}
+    for i, p in enumerate(ens.problems):
+        s = state(sizes[i], sizes[i], dtype, seed=sizes[i] + i % 3)
+        p.sol = s
+        starts[i] = s
+    gf.stepforward(ens, 4)
+    gf.stepforward(ens, 1)
+    for i in look:
+        ctor, kw = made[i]
+        single = ctor(gf.GPU(), **kw)
+        single.sol = starts[i]
+        gf.stepforward(single, 5)
+        assert rel(ens[i].sol, single.sol) < tol, (i, sizes[i])
