@@ -887,7 +887,10 @@ struct Ctx final : CtxBase {
     if (split[0] && ystage_built(d.ny, p, 3, cpw)) return 3;
     return ystage_built(d.ny, p, 1, cpw) ? 1 : 0;
   }
-  bool ypass_fusable() const { return ypass_groups() > 0; }
+  // the fixed-schedule problems: layers, and columns that are not a power of two long (one-layer
+  // MultiLayerQG problems are not fused: their drag reads a stage state that the fused pass does not store)
+  bool ypass_layers() const { return !tunable() && (nl > 1 || d.model != GF_MODEL_MLQG) && ylayers_built(nl, d.ny); }
+  bool ypass_fusable() const { return ypass_groups() > 0 || ypass_layers(); }
   // One stage of a run of stages on stream st: K1 unless the stage before has left its fields (first),
   // the x pass, then K3, or with fuse the fused y pass, without its second half in the last stage.
   void stage_launch(K1Args<T>& a, const K2Args<T>& b, K3Args<T>& c, bool fuse, bool first, bool last, hipStream_t st) {
@@ -895,7 +898,8 @@ struct Ctx final : CtxBase {
     if (first) { rec(0, true); launch_k1<T>(d.ny, a, st); rec(0, false); }
     rec(1, true); launch_k2<T>(d.nx, b, st); rec(1, false);
     if (last) a.ncols = 0;
-    if (fuse) launch_ystage<T>(d.ny, ypass_groups(), c, a, st);
+    if (fuse && ypass_layers()) launch_ylayers<T>(d.ny, c, a, st);
+    else if (fuse) launch_ystage<T>(d.ny, ypass_groups(), c, a, st);
     else { rec(2, true); launch_k3<T>(d.ny, c, st); rec(2, false); }
   }
 
@@ -960,7 +964,7 @@ struct Ctx final : CtxBase {
       for (auto& ge : gexec) if (ge) { HIPCHECK(hipStreamSynchronize(stream)); (void)dw::exec_destroy(ge); ge = nullptr; }
   }
   void get_schedule(int* p) const override {
-    for (int k = 0; k < 3; ++k) p[k] = sched[k] ? sched[k] : (nl == 1 ? sched_default(sched_len(k)) : (d.ny >= 32 && k != 1 ? (d.ny >= 4096 ? 8 : 4) : sched_default(sched_len(k))));
+    for (int k = 0; k < 3; ++k) p[k] = sched[k] ? sched[k] : (nl == 1 ? sched_default(sched_len(k)) : (d.ny >= 32 && k != 1 ? (d.ny >= 4096 ? 8 : d.ny <= 512 ? ylayers_p(pow2_ceil(d.ny)) : 4) : sched_default(sched_len(k))));
   }
   // Times whole steps under every offered schedule -- P in {4, 8, 16} for each of K1, K2, K3,
   // the K1 and K3 splits on or off and the K2 split 0, 1 or 2, up to 324 combinations -- in two

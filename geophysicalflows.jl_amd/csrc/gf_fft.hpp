@@ -342,7 +342,7 @@ __device__ __forceinline__ void fft_forward(cplx<T> (&v)[C][P], cplx<T>* __restr
 // of five LDS reads (four shared by the lanes) and 8 FMAs, where the plain sum of P outputs took
 // P n complex products of two reads each (n = 126: 31 steps against 504), and fewer roundings.
 // lds: 2 N slots; roots (LDS): exp(-2 pi i j/m), then exp(-2 pi i j/n), j < m.
-template <typename T, int N, int P>
+template <typename T, int N, int P, int X = X_FULL>
 __device__ __forceinline__ void dft_even(cplx<T> (&v)[1][P], cplx<T>* __restrict__ lds, int t, int n,
                                          const cplx<T>* __restrict__ roots) {
   static_assert(P == 4, "each thread forms the outputs of one k");
@@ -352,7 +352,7 @@ __device__ __forceinline__ void dft_even(cplx<T> (&v)[1][P], cplx<T>* __restrict
 #pragma unroll
   for (int q = 0; q < P; ++q)
     if (t + TPT * q < n) lds[t + TPT * q] = v[0][q];
-  __syncthreads();
+  xbarrier<X>();
   if (t < jm) {
     const int j = t + 1;
     const cplx<T> x0 = lds[j], x1 = lds[j + m], x2 = lds[m - j], x3 = lds[n - j];
@@ -371,7 +371,7 @@ __device__ __forceinline__ void dft_even(cplx<T> (&v)[1][P], cplx<T>* __restrict
     z0 = (t & 1) ? z0 - h0 : z0 + h0;
     z1 = (t & 1) ? z1 - h1 : z1 + h1;
   }
-  __syncthreads();
+  xbarrier<X>();
   cplx<T> c0 = z0, c1 = z1, d0 = mk((T)0, (T)0), d1 = d0;
   const bool mine = t <= m / 2;
   int idx = mine ? t : 0;
@@ -395,10 +395,10 @@ __device__ __forceinline__ void dft_even(cplx<T> (&v)[1][P], cplx<T>* __restrict
       lds[2 * (m - k) + 1] = mk(c1.re + d1.im, c1.im - d1.re);
     }
   }
-  __syncthreads();
+  xbarrier<X>();
 #pragma unroll
   for (int q = 0; q < P; ++q) v[0][q] = t + TPT * q < n ? lds[t + TPT * q] : mk((T)0, (T)0);
-  __syncthreads();                                   // lds is free again for the caller
+  xbarrier<X>();                                   // lds is free again for the caller
 }
 
 }  // namespace gf

@@ -291,6 +291,7 @@ template <typename T> void launch_k3(int ny, const K3Args<T>& a, hipStream_t s);
 // K3 of the stage c, then K1 (args a) of the next evaluation, on the same columns (groups 1 or 3);
 // a.ncols = 0: the stage alone
 template <typename T> void launch_ystage(int ny, int groups, const K3Args<T>& c, const K1Args<T>& a, hipStream_t s);
+template <typename T> void launch_ylayers(int ny, const K3Args<T>& c, const K1Args<T>& a, hipStream_t s);
 template <typename T> void launch_to_julia(const Geo<T>& g, const cplx<T>* src, cplx<T>* dst, int nl, hipStream_t s);
 template <typename T> void launch_from_julia(const Geo<T>& g, const cplx<T>* src, cplx<T>* dst, int nl, hipStream_t s);
 template <typename T> void launch_mask(const Geo<T>& g, cplx<T>* sol, int nl, hipStream_t s);
@@ -321,6 +322,13 @@ constexpr bool ystage_built(int n, int p, int ng, int cpw) {
   if (n < 32 || n > 4096 || (cpw == 1 && !k3_single_column(n, p))) return false;
   if (ng == 3) return n <= 1024 && (p == 4 || p == 8) && 3 * cpw * (n / p) <= 1024;
   return n >= 1024 && ((p == 4 && n == 1024) || p == 8 || (p == 16 && n == 4096));
+}
+// The fused y pass of short columns (gf_ylayers_impl.hpp), a wave per transform: 2 to 5 layers up to 512 points,
+// and single-layer problems whose columns are not a power of two long; its points per thread.
+constexpr int ylayers_p(int n) { return n >= 512 ? 8 : 4; }
+inline bool ylayers_built(int nl, int ny) {
+  const int n = pow2_ceil(ny);
+  return nl == 1 ? !is_pow2(ny) && n <= GEN_MAX : nl <= 5 && n >= 32 && n <= 512;
 }
 // Workgroups of a launch with G column pairs per workgroup over ncols columns; with quads and
 // G = 1, a multiple of 16 (pair_of_block puts the two pairs of a block on one XCD).

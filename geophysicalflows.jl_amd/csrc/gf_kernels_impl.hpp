@@ -165,11 +165,11 @@ __device__ __forceinline__ void load_y_twiddles(cplx<T>* __restrict__ tw, const 
   }
 }
 // the y-direction transform of a column of ny points held as fft_forward holds them
-template <typename T, int NY, int P, bool FR, bool GEN>
+template <typename T, int NY, int P, bool FR, bool GEN, int X = X_FULL>
 __device__ __forceinline__ void y_transform(cplx<T> (&w)[1][P], cplx<T>* __restrict__ L, int t,
                                             const cplx<T>* __restrict__ tw, int ny) {
-  if constexpr (GEN) dft_even<T, NY, P>(w, L, t, ny, tw);
-  else fft_forward<T, NY, P, 1, FR>(w, L, t, tw);
+  if constexpr (GEN) dft_even<T, NY, P, X>(w, L, t, ny, tw);
+  else fft_forward<T, NY, P, 1, FR, X>(w, L, t, tw);
 }
 // the column length the y-pass kernels index with
 template <int NY, bool GEN, typename T> __device__ __forceinline__ int ycol(const Geo<T>& g) {
@@ -1593,11 +1593,12 @@ template <int N> struct PCand {
     return p == 4 ? (N >= 16 && N <= 2048) : (p == 8 ? N >= 32 : (p == 16 ? N >= 1024 : false));
   }
 };
-// Points per thread of the multi-layer y passes: 4 (more, shorter transforms) up to 2048, 8 at
-// 4096 (a column pair of 4096 points at 4 per thread would need 2048 threads)
+// Points per thread of the multi-layer y passes: as the fused pass that runs between them where there is one
+// (ylayers_p), else 4 (more, shorter transforms) up to 2048 and 8 at 4096 (a column pair of 4096 points at
+// 4 per thread would need 2048 threads)
 // (column lengths that are not powers of two: 4, as dft_even needs)
 constexpr int PGEN = 4;
-template <int N> struct PML { static constexpr int P = N >= 4096 ? 8 : (N >= 32 ? 4 : PY<N>::P); };
+template <int N> struct PML { static constexpr int P = N >= 4096 ? 8 : (N >= 32 && N <= 512 ? ylayers_p(N) : (N >= 32 ? 4 : PY<N>::P)); };
 
 // ... and of their x pass
 template <int N> struct PMX { static constexpr int P = (N == 512 || N == 1024) ? 8 : 4; };

@@ -113,3 +113,36 @@ def test_both_ensemble_forms_match_members_stepped_alone(gf, counts, stepper, dt
         single.sol = starts[i]
         gf.stepforward(single, 5)
         assert rel(ens[i].sol, single.sol) < tol, (i, sizes[i])
+
+
+@pytest.mark.parametrize("nl,nx,ny", [(2, 32, 32), (3, 64, 64), (2, 32, 128), (4, 32, 256), (5, 32, 512), (3, 64, 512), (2, 18, 30), (5, 32, 34),
+                                      (3, 66, 62), (2, 128, 126), (4, 30, 254), (6, 32, 32), (2, 32, 16), (1, 64, 18), (1, 66, 250), (1, 22, 126)])
+@pytest.mark.parametrize("stepper,linear", [("ETDRK4", False), ("FilteredRK4", False), ("AB3", False), ("ETDRK4", True)])
+def test_fused_layers_and_ragged_columns_give_the_bits_of_the_separate_kernels(gf, nl, nx, ny, stepper, linear):
+    # multi-layer problems (2 to 5 layers are fused, 6 are not) with drag, ring forcing and topography, and
+    # TwoDNS / SingleLayerQG with columns that are not a power of two long
+    lib = gf._lib.lib
+    ring = gf.RingForcing(4.0, 1.5, 0.1, seed=7)
+    kw = dict(nx=nx, ny=ny, Ly=2 * np.pi * ny / nx, dt=1e-4, stepper=stepper)
+    eta = 0.1 * np.random.default_rng(1).standard_normal((ny, nx))
+    if nl > 1:
+        H = np.ones(nl) / nl
+        make = [lambda T: gf.MultiLayerQG.Problem(nl, gf.GPU(), f0=1.0, β=1.0, μ=0.2, ν=1e-6, U=0.1 * np.arange(nl), H=H,
+                                                  b=-1.0 - np.arange(nl) / nl, eta=eta, calcFq=ring, linear=linear, T=T, **kw)]
+    elif linear:
+        pytest.skip("one layer here is TwoDNS or SingleLayerQG")
+    else:
+        make = [lambda T: gf.TwoDNavierStokes.Problem(gf.GPU(), ν=1e-6, calcF=ring, T=T, **kw),
+                lambda T: gf.SingleLayerQG.Problem(gf.GPU(), β=2.0, μ=0.1, eta=eta, deformation_radius=0.7, T=T, **kw)]
+    for mk in make:
+        for T in (np.float64, np.float32):
+            sols = []
+            for timed in (0, 1):
+                p = mk(T)
+                s = state(ny, nx, T)
+                p.sol = s if nl == 1 else np.stack([s * (1 - 0.1 * j) for j in range(nl)])
+                assert lib.gf_timing(p._ctx, timed) == 0
+                gf.stepforward(p, 4)
+                gf.stepforward(p, 1)
+                sols.append(p.sol)
+            assert np.isfinite(sols[0]).all() and np.array_equal(sols[0], sols[1])
