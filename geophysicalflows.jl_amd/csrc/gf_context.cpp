@@ -1515,7 +1515,7 @@ struct Ctx final : CtxBase {
     adj_mixed.alloc(sizeof(C) * fsz * 5);
     adj_flux.alloc(sizeof(C) * fsz * 3);
     for (DevBuf* b : {&lamb, &l0b, &l1b, &lN1b, &lN2b, &lN3b}) b->alloc(sizeof(C) * fsz);
-    ka3_blocks = adj_blocks<double>(d.ny, g.kmax);
+    ka3_blocks = std::max(adj_blocks<double>(d.ny, g.kmax), adj_group_built(d.ny) ? adj_group_blocks(d.ny, g.kmax) : 0);
     nu_part.alloc(sizeof(double) * ka3_blocks);
     // dJ/dnu tables: d(coefficient)/dL times dL/dnu = -Krsq^nnu (0 at k = 0)
     const int ny = d.ny, nkr = g.nkr;
@@ -1572,38 +1572,55 @@ struct Ctx final : CtxBase {
     HIPCHECK(hipGetLastError());
   }
 
-  // adjoint of the step taped in slot i of tape tp: lamb (lambda of the new state) -> lambda of s0
-  void adjoint_step(long i, bool want_nu, int tp = 0) {
+  // argument blocks of the adjoint of stage `stage` of the step taped in slot i of tape tp
+  void adjoint_args(long i, int stage, bool want_nu, int tp, AdjK1Args<T>& a, AdjK2Args<T>& b, AdjK3Args<T>& k) {
+    a = AdjK1Args<T>{};
+    a.g = g; a.stage = stage;
+    a.s0 = slot(i, 0, tp); a.N1 = slot(i, 1, tp); a.N2 = slot(i, 2, tp); a.N3 = slot(i, 3, tp);
+    a.E2 = (const T*)coef[0].p; a.Z = (const T*)coef[1].p;
+    a.x = stage == 4 ? lamb.as<C>() : stage == 3 ? lN3b.as<C>() : stage == 2 ? lN2b.as<C>() : lN1b.as<C>();
+    a.lamc = stage == 4 ? (const T*)coef[5].p : nullptr;
+    a.out = adj_mixed.as<C>(); a.fstride = fsz; a.ncols = g.kmax; a.tw = twy.as<C>();
+    a.fsplit = split[0];   // the forward problem's tuned workgroup splits
+    b = AdjK2Args<T>{};
+    b.g = g; b.in = adj_mixed.as<C>(); b.fstride = fsz; b.kin = g.kmax;
+    b.out = adj_flux.as<C>(); b.ostride = fsz; b.kout = g.kmax; b.tw = twx.as<C>();
+    b.hsplit = split[1] != 0;
+    k = AdjK3Args<T>{};
+    k.g = g; k.in = adj_flux.as<C>(); k.fstride = fsz; k.ncols = g.kmax; k.stage = stage;
+    k.lam = lamb.as<C>(); k.l0 = l0b.as<C>(); k.l1 = l1b.as<C>();
+    k.lN1 = lN1b.as<C>(); k.lN2 = lN2b.as<C>(); k.lN3 = lN3b.as<C>();
+    k.E2 = (const T*)coef[0].p; k.Z = (const T*)coef[1].p; k.E = (const T*)coef[2].p;
+    k.Al = (const T*)coef[3].p; k.Be = (const T*)coef[4].p;
+    k.dE = dtab[0].as<T>(); k.dE2 = dtab[1].as<T>(); k.dZ = dtab[2].as<T>();
+    k.dA = dtab[3].as<T>(); k.dB = dtab[4].as<T>(); k.dG = dtab[5].as<T>();
+    k.s0 = slot(i, 0, tp);
+    k.N1 = slot(i, 1, tp); k.N2 = slot(i, 2, tp); k.N3 = slot(i, 3, tp); k.N4 = slot(i, 4, tp);
+    k.nu_part = want_nu ? nu_part.as<T>() : nullptr;
+    k.tw = twy.as<C>();
+  }
+  // adjoint of the n steps taped in tape tp, last to first: lamb (lambda of the last new state) -> lambda of
+  // the first step's input
+  void adjoint_sweep(long n, bool want_nu, int tp) {
     if constexpr (std::is_same<T, double>::value) {
-      for (int stage = 4; stage >= 1; --stage) {
-        AdjK1Args<T> a{};
-        a.g = g; a.stage = stage;
-        a.s0 = slot(i, 0, tp); a.N1 = slot(i, 1, tp); a.N2 = slot(i, 2, tp); a.N3 = slot(i, 3, tp);
-        a.E2 = (const T*)coef[0].p; a.Z = (const T*)coef[1].p;
-        a.x = stage == 4 ? lamb.as<C>() : stage == 3 ? lN3b.as<C>() : stage == 2 ? lN2b.as<C>() : lN1b.as<C>();
-        a.lamc = stage == 4 ? (const T*)coef[5].p : nullptr;
-        a.out = adj_mixed.as<C>(); a.fstride = fsz; a.ncols = g.kmax; a.tw = twy.as<C>();
-        a.fsplit = split[0];   // the forward problem's tuned workgroup splits
-        AdjK2Args<T> b{};
-        b.g = g; b.in = adj_mixed.as<C>(); b.fstride = fsz; b.kin = g.kmax;
-        b.out = adj_flux.as<C>(); b.ostride = fsz; b.kout = g.kmax; b.tw = twx.as<C>();
-        b.hsplit = split[1] != 0;
-        AdjK3Args<T> k{};
-        k.g = g; k.in = adj_flux.as<C>(); k.fstride = fsz; k.ncols = g.kmax; k.stage = stage;
-        k.lam = lamb.as<C>(); k.l0 = l0b.as<C>(); k.l1 = l1b.as<C>();
-        k.lN1 = lN1b.as<C>(); k.lN2 = lN2b.as<C>(); k.lN3 = lN3b.as<C>();
-        k.E2 = (const T*)coef[0].p; k.Z = (const T*)coef[1].p; k.E = (const T*)coef[2].p;
-        k.Al = (const T*)coef[3].p; k.Be = (const T*)coef[4].p;
-        k.dE = dtab[0].as<T>(); k.dE2 = dtab[1].as<T>(); k.dZ = dtab[2].as<T>();
-        k.dA = dtab[3].as<T>(); k.dB = dtab[4].as<T>(); k.dG = dtab[5].as<T>();
-        k.s0 = slot(i, 0, tp);
-        k.N1 = slot(i, 1, tp); k.N2 = slot(i, 2, tp); k.N3 = slot(i, 3, tp); k.N4 = slot(i, 4, tp);
-        k.nu_part = want_nu ? nu_part.as<T>() : nullptr;
-        k.tw = twy.as<C>();
-        rec(0, true); launch_adj<T>(1, d.ny, &a, stream); rec(0, false);
-        rec(1, true); launch_adj<T>(2, d.nx, &b, stream); rec(1, false);
-        rec(2, true); launch_adj<T>(3, d.ny, &k, stream); rec(2, false);
-      }
+      AdjK1Args<T> a; AdjK2Args<T> b; AdjK3Args<T> k;
+      const bool two = adj_group_built(d.ny) && !tm.on;   // (the kernels are timed one by one)
+      for (long i = n - 1; i >= 0; --i)
+        for (int stage = 4; stage >= 1; --stage) {
+          adjoint_args(i, stage, want_nu, tp, a, b, k);
+          if (two) {
+            if (i == n - 1 && stage == 4) launch_adj_y(d.ny, k, a, 0, stream);
+            launch_adj_x(d.nx, b, stream);
+            const bool last = i == 0 && stage == 1;
+            AdjK2Args<T> bn; AdjK3Args<T> kn;
+            if (!last) adjoint_args(stage > 1 ? i : i - 1, stage > 1 ? stage - 1 : 4, want_nu, tp, a, bn, kn);
+            launch_adj_y(d.ny, k, a, last ? 2 : 1, stream);
+            continue;
+          }
+          rec(0, true); launch_adj<T>(1, d.ny, &a, stream); rec(0, false);
+          rec(1, true); launch_adj<T>(2, d.nx, &b, stream); rec(1, false);
+          rec(2, true); launch_adj<T>(3, d.ny, &k, stream); rec(2, false);
+        }
       HIPCHECK(hipGetLastError());
     }
   }
@@ -1720,7 +1737,7 @@ struct Ctx final : CtxBase {
           HIPCHECK(hipMemcpyAsync(slot(0, 0, tp), ckpts.as<C>() + s * kstride(), kb, hipMemcpyDeviceToDevice, stream));
           tape_steps(n, tp, stream);
         }
-        for (long i = n - 1; i >= 0; --i) adjoint_step(i, dnu != nullptr, tp);
+        adjoint_sweep(n, dnu != nullptr, tp);
       }
       for (long s = nseg - 1; s >= 0 && pipe; --s) {
         const int tp = tape_of(s);
@@ -1736,7 +1753,7 @@ struct Ctx final : CtxBase {
         }
         if (s < resident) HIPCHECK(hipStreamWaitEvent(stream, rec_done[tp], 0));
         const long n = len(s);
-        for (long i = n - 1; i >= 0; --i) adjoint_step(i, dnu != nullptr, tp);
+        adjoint_sweep(n, dnu != nullptr, tp);
         HIPCHECK(hipEventRecord(adj_done[tp], stream));
       }
       // dJ/dzeta0 = N irfft2(Z M lambda_0 / w)

@@ -224,6 +224,13 @@ template <typename T> void launch_adj(int k, int n, const void* args, hipStream_
 // workgroups of KA3 (and KA1) for ncols columns at size n
 template <typename T> int adj_blocks(int n, int ncols);
 
+// The two-launch form of grids it is built for (gf_adj_group.hip): KA2, and KA3 of the stage k with KA1 of the
+// next (a): mode 0 KA1 alone, 1 both, 2 KA3 alone; the workgroups (nu_part slots) of the latter.
+bool adj_group_built(int n);
+int adj_group_blocks(int n, int ncols);
+void launch_adj_x(int n, const AdjK2Args<double>& b, hipStream_t s);
+void launch_adj_y(int n, const AdjK3Args<double>& k, const AdjK1Args<double>& a, int mode, hipStream_t s);
+
 // Domain-averaged diagnostics (gf_diag.hip); kinds as GF_DIAG_* in include/gf.h.
 enum DiagKind {
   DIAG_ENERGY = 0, DIAG_KINETIC_ENERGY = 1, DIAG_POTENTIAL_ENERGY = 2, DIAG_ENSTROPHY = 3,

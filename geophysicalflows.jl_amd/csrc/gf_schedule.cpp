@@ -126,6 +126,16 @@ bool sched_by_length(const SchedKey& key, Sched& out) {
   const Sched* col = best(key[3]);
   const Sched* row = best(key[2]);
   if (!col && !row) return false;
+  // one length shorter than the table goes: the form of the next longer one there is, where every
+  // radix it names is offered
+  auto longer = [&](int n, const Sched*& e, int k0, int k1) {
+    for (int m = 2 * n; !e && m <= 4096; m *= 2) e = best(m);
+    if (!e) return;
+    for (int k : {k0, k1})
+      if (!offered(n, e->p[k])) { e = nullptr; return; }
+  };
+  if (!row) longer(key[2], row, 1, 1);
+  if (!col) longer(key[3], col, 0, 2);
   out = Sched{};
   if (col) {
     out.p[0] = col->p[0]; out.p[2] = col->p[2];

@@ -19,7 +19,8 @@ bool sched_lookup(const SchedKey& key, Sched& out);
 // For a single-layer problem without an entry of its own: K1 and K3 transform columns of ny points
 // and K2 rows of nx, so each takes what the table has for square grids of that length, of the same
 // model and precision if there is one, else of the same precision, else any. False where the table
-// has no square grid of either length (the built-in choice then).
+// has no square grid of either length (the built-in choice then); where it has one of them, the other
+// takes the next longer length's.
 bool sched_by_length(const SchedKey& key, Sched& out);
 void sched_store(const SchedKey& key, const Sched& s);
 void sched_clear();

@@ -146,3 +146,20 @@ def test_fused_layers_and_ragged_columns_give_the_bits_of_the_separate_kernels(g
                 gf.stepforward(p, 1)
                 sols.append(p.sol)
             assert np.isfinite(sols[0]).all() and np.array_equal(sols[0], sols[1])
+
+
+@pytest.mark.parametrize("n", [32, 64, 128, 256, 512, 1024])
+def test_two_launch_adjoint_matches_the_separate_kernels(gf, n):
+    # per-kernel timing runs KA1, KA2 and KA3 one by one (1024^2 always does); the two forms sum the same
+    # terms of 5 steps in other orders: 1e-12 relative
+    z = 0.3 * np.random.default_rng(n).standard_normal((n, n))
+    target = 0.1 * np.random.default_rng(n + 1).standard_normal((n, n))
+    got = []
+    for timed in (0, 1):
+        p = gf.TwoDNavierStokes.Problem(gf.GPU(), nx=n, ν=1e-3, nν=1, dt=1e-3, stepper="ETDRK4")
+        gf.TwoDNavierStokes.set_ζ(p, z)
+        assert gf._lib.lib.gf_timing(p._ctx, timed) == 0
+        got.append(gf.TwoDNavierStokes.adjoint_gradient(p, target, 5, 2))
+    (J0, g0, nu0), (J1, g1, nu1) = got
+    assert abs(J0 - J1) <= 1e-13 * abs(J1) and abs(nu0 - nu1) <= 1e-11 * abs(nu1)
+    assert rel(g0, g1) < 1e-12
