@@ -90,7 +90,10 @@ template <typename T> struct Coef {
   // elements i and i + 1 (every table carries 16 bytes of padding), the second then unused. With
   // a branch on the kind between a load and its use, the compiler waited for each coefficient
   // before issuing the next load.
-  __device__ __forceinline__ cplx<T> get(uint32_t i) const {
+  // CP: the table's kind where the caller knows it (0 real, 1 complex), -1 to ask
+  template <int CP> __device__ __forceinline__ cplx<T> get(uint32_t i) const {
+    if constexpr (CP == 0) return mk(at(reinterpret_cast<const T*>(p), i), (T)0);
+    if constexpr (CP == 1) return at(reinterpret_cast<const cplx<T>*>(p), i);
     const T* e = reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) +
                                             i * (uint32_t)(cplx_ ? sizeof(cplx<T>) : sizeof(T)));
     return mk(e[0], e[1]);
@@ -1245,10 +1248,10 @@ template <typename T> struct StagePoint {
 // the stages compute for every lane and store only where kept: loads under a branch on kept made the
 // compiler wait for each before issuing the next.
 template <typename T> struct StageIn { cplx<T> sol, x, y, z, k[4]; T filter; };
-template <typename T>
+template <typename T, int CP = -1>
 __device__ __forceinline__ StageIn<T> stage_load(const K3Args<T>& a, int epi, const StagePoint<T>& p) {
   StageIn<T> in{};
-  auto coef = [&](const void* c) { return Coef<T>{c, a.ccplx}.get(p.ci); };
+  auto coef = [&](const void* c) { return Coef<T>{c, a.ccplx}.template get<CP>(p.ci); };
   in.sol = at(a.sol, p.ix);
   switch (epi) {
     case E_ETD3:
@@ -1285,11 +1288,12 @@ __device__ __forceinline__ StageIn<T> stage_load(const K3Args<T>& a, int epi, co
 }
 // N of one point from its transformed fluxes Av, Bv, then the stage `epi`.  Returns the state the
 // next calcN! reads there (what kept points store).  NEXT: the caller hands that state on itself, so the
-// ETDRK4 stages 2 and 3, whose state nothing else reads, do not store it.
-template <typename T, int NL, bool ML1, bool NEXT>
+// ETDRK4 stages 2 and 3, whose state nothing else reads, do not store it.  LATE: the caller stores the new
+// state of a step's last stage itself, and gets it whether kept or not.
+template <typename T, int NL, bool ML1, bool NEXT, int CP = -1, bool LATE = false>
 __device__ __forceinline__ cplx<T> stage_point(const K3Args<T>& a, int epi, const StagePoint<T>& p, const StageIn<T>& in, bool kept,
                                                int jl, T kv, T lv, cplx<T> Av, cplx<T> Bv, cplx<T> psin, const cplx<T>* noise, bool& bad) {
-  const int kr = p.kr, l = p.l, ny = p.ny, cp = a.ccplx;
+  const int kr = p.kr, l = p.l, ny = p.ny, cp = CP >= 0 ? CP : a.ccplx;
   const uint32_t idx = p.idx, ix = p.ix;
   cplx<T> N;
   if (a.apply_kr) {
@@ -1353,7 +1357,7 @@ __device__ __forceinline__ cplx<T> stage_point(const K3Args<T>& a, int epi, cons
       r = coef_fma(cp, in.k[2], mk((T)2 * in.z.re, (T)2 * in.z.im), r);
       r = coef_fma(cp, in.k[3], N, r);
       if (a.filter) r = rmul(in.filter, r);
-      at(a.sol_out != nullptr ? a.sol_out : a.sol, ix) = r;
+      if constexpr (!LATE) at(a.sol_out != nullptr ? a.sol_out : a.sol, ix) = r;
       bad |= !finite(r);
       break;
     case E_RK1:
@@ -1378,14 +1382,14 @@ __device__ __forceinline__ cplx<T> stage_point(const K3Args<T>& a, int epi, cons
         const cplx<T> acc = mk(in.y.re + R.re / (T)6, in.y.im + R.im / (T)6);
         r = rfma(a.dt, acc, sv);
         if (a.filter) r = rmul(in.filter, r);
-        at(a.sol, ix) = r;
+        if constexpr (!LATE) at(a.sol, ix) = r;
         bad |= !finite(r);
       }
     } break;
     case E_FE:
       r = rfma(a.dt, coef_fma(cp, in.k[0], sv, N), sv);
       if (a.filter) r = rmul(in.filter, r);
-      at(a.sol, ix) = r;
+      if constexpr (!LATE) at(a.sol, ix) = r;
       bad |= !finite(r);
       break;
     case E_AB3: {
@@ -1406,7 +1410,7 @@ __device__ __forceinline__ cplx<T> stage_point(const K3Args<T>& a, int epi, cons
     } break;
     default: break;
   }
-  return kept ? r : czero<T>();
+  return kept || LATE ? r : czero<T>();
 }
 
 // Body of K3 for block blk of column pairs (CPW = 2, G pairs per workgroup) or, with CPW = 1,

@@ -48,6 +48,7 @@ __device__ __forceinline__ void ystage_body(const K3Args<T>& c, const K1Args<T>&
   constexpr int TPT = Y::TPT, G = Y::G, GT = Y::GT, X = Y::X, PG = XPad<T>::G, BUF = YLds<T, NY, P, NG, CPW>::BUF;
   constexpr bool FR = NG == 1 && sizeof(T) == 8 && NY >= 2048;
   constexpr bool TIGHT = Y::TIGHT;
+  constexpr int CP = MODEL == M_TWODNS ? 0 : 1;       // real or complex coefficient tables
   const Geo<T>& g = c.g;
   const int grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / GT);
   const int tid = (int)threadIdx.x % GT;
@@ -101,7 +102,7 @@ __device__ __forceinline__ void ystage_body(const K3Args<T>& c, const K1Args<T>&
   if constexpr (AHEAD) {
 #pragma unroll
     for (int i = 0; i < Y::QN; ++i)
-      in[i] = stage_load<T>(c, epi, StagePoint<T>(c, krl, mine(i) ? row(i) : t, NY, 0u));
+      in[i] = stage_load<T, CP>(c, epi, StagePoint<T>(c, krl, mine(i) ? row(i) : t, NY, 0u));
   }
   // ring forcing: this thread's terms, read back by it in the stage (k3_body)
   if (c.sqrt_spec != nullptr && active && kr <= c.fkx) {
@@ -123,17 +124,39 @@ __device__ __forceinline__ void ystage_body(const K3Args<T>& c, const K1Args<T>&
 
   bool bad = false;
   if constexpr (NG == 1) {
+    // A wait for reads issued after a store waits for the store too (both count in vmcnt), and row by row
+    // that chained the P stores' latencies. So each mode's reads are issued before the mode before it stores
+    // (PIPE), and the last stage of a step, whose reads would take too many registers for that, stores its new
+    // state after the loop (LATE). 2048^2 FP64: ETDRK4 stages 1 and 4 45 and 47 -> 40 and 42 us.
+    constexpr bool LATE = EPI == E_ETD4 || EPI == E_RK4 || EPI == E_FE, PIPE = !LATE && !TIGHT;
+    // (a row that is not stepped reads the column's first one)
+    auto stepped = [&](int l) { return (kept_l(g, l) && kr < g.kmax) || c.full; };
+    auto read = [&](int q) {
+      const int l = t + TPT * q;
+      return stage_load<T, CP>(c, epi, StagePoint<T>(c, krl, stepped(l) ? l : 0, NY, 0u));
+    };
+    StageIn<T> next;
+    if constexpr (PIPE) next = read(0);
 #pragma unroll
     for (int q = 0; q < P; ++q) {
       const int l = t + TPT * q;
       const bool kept = kept_l(g, l) && kr < g.kmax;
+      const StageIn<T> one = PIPE ? next : read(q);
+      if (PIPE && q + 1 < P) next = read(q + 1);
       sv[q] = czero<T>();
-      if (active && (kept || c.full)) {
-        const StagePoint<T> pt(c, kr, l, NY, 0u);
-        const StageIn<T> one = stage_load<T>(c, epi, pt);
-        sv[q] = stage_point<T, 1, false, true>(c, epi, pt, one, kept, 0, kv, lwave(g, l), w[0][q], w1[0][q], czero<T>(), c.noise, bad);
-      }
+      if (active && stepped(l))
+        sv[q] = stage_point<T, 1, false, true, CP, LATE>(c, epi, StagePoint<T>(c, kr, l, NY, 0u), one, kept, 0, kv, lwave(g, l), w[0][q], w1[0][q],
+                                                         czero<T>(), c.noise, bad);
       if constexpr (P >= 8) __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (LATE) {
+      cplx<T>* o = EPI == E_ETD4 && c.sol_out != nullptr ? c.sol_out : c.sol;
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        const int l = t + TPT * q;
+        if (active && stepped(l)) at(o, boff32(kr, l, NY)) = sv[q];
+        if (!(kept_l(g, l) && kr < g.kmax)) sv[q] = czero<T>();
+      }
     }
   } else {
     // the transformed fluxes cross groups in buffers 0 and 1, the new modes come back in buffer 2
@@ -154,8 +177,8 @@ __device__ __forceinline__ void ystage_body(const K3Args<T>& c, const K1Args<T>&
       cplx<T> r = czero<T>();
       if (active && (kept || c.full)) {
         const StagePoint<T> pt(c, kr, l, NY, 0u);
-        const StageIn<T> one = AHEAD ? in[AHEAD ? i : 0] : stage_load<T>(c, epi, pt);
-        r = stage_point<T, 1, false, true>(c, epi, pt, one, kept, 0, kv, lwave(g, l), A[s], B[s], czero<T>(), c.noise, bad);
+        const StageIn<T> one = AHEAD ? in[AHEAD ? i : 0] : stage_load<T, CP>(c, epi, pt);
+        r = stage_point<T, 1, false, true, CP>(c, epi, pt, one, kept, 0, kv, lwave(g, l), A[s], B[s], czero<T>(), c.noise, bad);
       }
       S[s] = r;
     }
