@@ -52,6 +52,8 @@ __device__ __forceinline__ void batch_body(const BatchItem<T>& it, int blk, cplx
     __syncthreads();
     if (!PLAIN && it.k2.mode == K2_ADVECT_FULL) {
       if constexpr (!PLAIN) k2_body<T, N, BATCH_P, BG::G2, K2_ADVECT_FULL, 1>(it.k2, blk, lds, tw);
+    } else if (!PLAIN && it.k2.mode == K2_ADVECT_Y) {
+      if constexpr (!PLAIN) k2_body<T, N, BATCH_P, BG::G2, K2_ADVECT_Y, 1>(it.k2, blk, lds, tw);
     } else {
       k2_body<T, N, BATCH_P, BG::G2, K2_ADVECT, 1>(it.k2, blk, lds, tw);
     }

@@ -33,23 +33,25 @@ template <typename T, int NG> size_t batch2_lds(int nmax) {
   return sizeof(cplx<T>) * (size_t)m;
 }
 
-template <typename T, int N, int NG, bool FULL>
+template <typename T, int N, int NG, int MODE>
 __device__ __forceinline__ void batch2_xn(const BatchItem<T>& it, int blk, cplx<T>* lds, cplx<T>* tw) {
   constexpr int P = Batch2<N, NG>::P;
   if constexpr (NG == 3) {
-    k2_group_body<T, N, P, FULL>(it.k2, blk, 0, lds, tw);
+    k2_group_body<T, N, P, MODE>(it.k2, blk, 0, lds, tw);
   } else {
     load_twiddles<T, N, P>(tw, it.k2.tw);
     xbarrier<X_WAVE>();
-    k2_body<T, N, P, K2P<N, P>::G, FULL ? K2_ADVECT_FULL : K2_ADVECT, 1, X_WAVE>(it.k2, blk, lds, tw);
+    k2_body<T, N, P, K2P<N, P>::G, MODE, 1, X_WAVE>(it.k2, blk, lds, tw);
   }
 }
 template <typename T, int N, int NG, bool PLAIN>
 __device__ __forceinline__ void batch2_x(const BatchItem<T>& it, int blk, cplx<T>* lds, cplx<T>* tw) {
   if (!PLAIN && it.k2.mode == K2_ADVECT_FULL) {
-    if constexpr (!PLAIN) batch2_xn<T, N, NG, true>(it, blk, lds, tw);
+    if constexpr (!PLAIN) batch2_xn<T, N, NG, K2_ADVECT_FULL>(it, blk, lds, tw);
+  } else if (!PLAIN && it.k2.mode == K2_ADVECT_Y) {
+    if constexpr (!PLAIN) batch2_xn<T, N, NG, K2_ADVECT_Y>(it, blk, lds, tw);
   } else {
-    batch2_xn<T, N, NG, false>(it, blk, lds, tw);
+    batch2_xn<T, N, NG, K2_ADVECT>(it, blk, lds, tw);
   }
 }
 template <typename T, int N, int NG>

@@ -637,9 +637,16 @@ struct Ctx final : CtxBase {
         std::vector<double> Uyy = spectral_op(U2, 2);
         std::vector<double> ex = spectral_op(etav, 0), ey = spectral_op(etav, 1);
         for (size_t i = 0; i < np; ++i) ey[i] -= Uyy[i];
-        upload_real(etax, ex); upload_real(etay, ey);
+        std::vector<double> Qy(ny, 0.0);
+        if (has_eta) { upload_real(etax, ex); upload_real(etay, ey); }
+        else {                                          // the same along x, up to its rounding: the mean
+          for (int y = 0; y < ny; ++y) {
+            for (int x = 0; x < nx; ++x) Qy[y] -= Uyy[(size_t)y * nx + x];
+            Qy[y] /= nx;
+          }
+        }
         upload_real(Uy, std::vector<double>(d.Uy, d.Uy + ny));
-        upload_real(Qy1, std::vector<double>(ny, 0.0));
+        upload_real(Qy1, Qy);
       }
       return;
     }
@@ -714,12 +721,16 @@ struct Ctx final : CtxBase {
         else q = q - Fp[j] * (Uj(j + 1) - Uj(j)) - Fm[j - 1] * (Uj(j - 1) - Uj(j));
         Qy[(size_t)j * ny + y] = q;
       }
+    const bool xdep = has_eta || d.topo_grad_x != 0;    // bottom layer's Qx, or a Qy that depends on x
+    if (!xdep) for (int y = 0; y < ny; ++y) Qy[(size_t)(n - 1) * ny + y] += d.topo_grad_y;
     upload_real(Uy, U);
     upload_real(Qy1, Qy);
-    std::vector<double> ex = has_eta ? spectral_op(etav, 0) : std::vector<double>(np, 0.0);
-    std::vector<double> ey = has_eta ? spectral_op(etav, 1) : std::vector<double>(np, 0.0);
-    for (size_t i = 0; i < np; ++i) { ex[i] += d.topo_grad_x; ey[i] += d.topo_grad_y; }
-    upload_real(etax, ex); upload_real(etay, ey);
+    if (xdep) {
+      std::vector<double> ex = has_eta ? spectral_op(etav, 0) : std::vector<double>(np, 0.0);
+      std::vector<double> ey = has_eta ? spectral_op(etav, 1) : std::vector<double>(np, 0.0);
+      for (size_t i = 0; i < np; ++i) { ex[i] += d.topo_grad_x; ey[i] += d.topo_grad_y; }
+      upload_real(etax, ex); upload_real(etay, ey);
+    }
   }
 
   bool filtered() const {
@@ -816,7 +827,7 @@ struct Ctx final : CtxBase {
     a.g = g; a.model = d.model; a.fieldset = FS_CALCN; a.sol = in; a.out = mixed.as<C>(); a.fstride = fsz;
     a.ncols = g.kmax; a.eb = eb; a.ell2inv = (T)ell2inv; a.sinv = sinv.as<T>(); a.tw = twy.as<C>();
     b = K2Args<T>{};
-    b.g = g; b.mode = advect_full ? K2_ADVECT_FULL : K2_ADVECT; b.in = mixed.as<C>(); b.fstride = fsz;
+    b.g = g; b.mode = advect_full ? (etax.p || d.linear ? K2_ADVECT_FULL : K2_ADVECT_Y) : K2_ADVECT; b.in = mixed.as<C>(); b.fstride = fsz;
     b.kin = g.kmax; b.eta = (d.model == GF_MODEL_SLQG && !advect_full && has_eta) ? eta.as<T>() : nullptr;
     b.Uy = Uy.as<T>(); b.Qy1 = Qy1.as<T>(); b.etax = etax.as<T>(); b.etay = etay.as<T>(); b.has_bg = advect_full;
     b.out = flux.as<C>(); b.ostride = fsz; b.kout = full ? g.nkr : g.kmax; b.tw = twx.as<C>();
@@ -1324,7 +1335,7 @@ struct Ctx final : CtxBase {
     if (k == 1) {
       double b = 3 * kmax * ny * cs * L + 2 * cols * ny * cs * L;
       if (d.model == GF_MODEL_SLQG && has_eta && !advect_full) b += (double)d.nx * ny * rs;
-      if (advect_full && has_eta) b += 2 * (double)d.nx * ny * rs;
+      if (etax.p) b += 2 * (double)d.nx * ny * rs;
       return b;
     }
     // K3: flux read + the average stage epilogue of the configured stepper

@@ -49,8 +49,10 @@ enum Field { F_U = 0, F_V = 1, F_Q = 2, F_PSI = 3, F_RAW = 4 };
 // (q, psi, u, v) for the QG models), FS_RAW = the state itself, unmasked.
 enum FieldSet { FS_CALCN = 0, FS_OUT = 1, FS_RAW = 2 };
 
-// K2 modes
-enum K2Mode { K2_ADVECT = 0, K2_INVERSE_OUT = 1, K2_FORWARD_IN = 2, K2_ADVECT_FULL = 3 };
+// K2 modes.  Background gradients that depend on y only (a U(y) or layers without topography) need no
+// transform of their own: (v Qy)^ = Qy v^ row by row (K2_ADVECT_Y); with Qx or a Qy that depends on x the
+// product u Qx + v Qy is transformed (K2_ADVECT_FULL, also the linearised equations).
+enum K2Mode { K2_ADVECT = 0, K2_INVERSE_OUT = 1, K2_FORWARD_IN = 2, K2_ADVECT_FULL = 3, K2_ADVECT_Y = 4 };
 
 // K3 epilogues
 enum Epi {
@@ -103,7 +105,7 @@ struct K2Args {
   long fstride;
   int kin;                  // kr < kin present in the input mixed fields
   const T* eta;             // SLQG: physical eta (x fastest), nullable
-  // advect-full (MLQG / SLQG varying U): per-layer U(y), Qy(y); bottom-layer Qx/Qy fields
+  // background (MLQG / SLQG varying U): per-layer U(y), Qy(y); bottom-layer Qx/Qy fields (K2_ADVECT_FULL)
   const T* Uy;              // nlayers*ny
   const T* Qy1;             // nlayers*ny
   const T* etax;            // ny*nx, bottom layer, nullable

@@ -428,17 +428,24 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
         }
       }
     }
-  } else if constexpr (MODE == K2_ADVECT) {
+  } else if constexpr (MODE == K2_ADVECT || MODE == K2_ADVECT_Y) {
     // ---- advection without background gradients: u, v, q -> u (q [+ eta]), v (q [+ eta]) ----
-    // (src/twodnavierstokes.jl:262-270, src/singlelayerqg.jl:368-375).  Every transform packs
+    // (src/twodnavierstokes.jl:262-270, src/singlelayerqg.jl:368-375), or with gradients that depend on y
+    // only (K2_ADVECT_Y): u += U, (-i kr (u q)^ - (v Qy)^, (v q)^) per layer
+    // (src/multilayerqg.jl:695-731), where (v Qy)^ is Qy v^ row by row: five transforms and the registers
+    // of K2_ADVECT (117 VGPRs at 2048, P = 8) instead of six and 240.  U(y) at 2048^2, against
+    // K2_ADVECT_FULL: FP64 68-72 -> 44 us, FP32 56 -> 34.  Every transform packs
     // the two rows of one field: inverse (q0 + i q1), (u0 + i u1), (v0 + i v1) and forward
     // (u0 q0 + i u1 q1), (v0 q0 + i v1 q1).  A phase thus reads and writes whole 64-byte pieces
     // (two rows of a column pair; with the workgroup's other row pair, whole 128-byte lines), and
     // only q stays live across phases.
-    static_assert(NL == 1, "K2_ADVECT serves single-layer models");
-    const cplx<T>* fu = a.in;
-    const cplx<T>* fv = a.in + a.fstride;
-    const cplx<T>* fq = a.in + 2 * a.fstride;
+    constexpr bool JET = MODE == K2_ADVECT_Y;
+    static_assert(NL == 1 || JET, "K2_ADVECT serves single-layer models");
+    const int jl = NL > 1 ? (int)blockIdx.y : 0;        // (a layer per workgroup row)
+    const cplx<T>* fu = a.in + (long)(3 * jl) * a.fstride;
+    const cplx<T>* fv = fu + a.fstride;
+    const cplx<T>* fq = fv + a.fstride;
+    cplx<T>* out = a.out + (long)(2 * jl) * a.ostride;
     auto load_rows = [&](const cplx<T>* f, cplx<T> (&w)[1][P]) {
       // Only points k <= NX/2 are read from memory. The Hermitian half k > NX/2 is the packed
       // value of the mirror NX - k, conj(conj A + i conj B): the loading lane leaves it in LDS slot
@@ -476,8 +483,20 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
       load_rows(f, w);
       fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2), X>(w, L, t, tw);             // row y0 = Re, row y0 + 1 = -Im
     };
-    auto forward_rows = [&](cplx<T>* o, cplx<T> (&w)[1][P]) {
+    auto forward_rows = [&](cplx<T>* o, cplx<T> (&w)[1][P], bool gradient) {
       fft_forward<T, NX, P, 1, (NX >= FreshFrom<T>::k2), X>(w, L, t, tw);             // of (row y0 + i row y0 + 1)
+      // (v Qy)^ = Qy v^: the spectrum K1 left, which these lanes read before (times NX, as every
+      // product here)
+      cplx<T> c0[JET ? MAXI : 1], c1[JET ? MAXI : 1];
+      if (JET && gradient) {
+        const T e0 = active ? (T)NX * a.Qy1[jl * ny + y0] : (T)0, e1 = active ? (T)NX * a.Qy1[jl * ny + y0 + 1] : (T)0;
+#pragma unroll
+        for (int i = 0; i < (JET ? MAXI : 1); ++i) {
+          const int kr = t + i * TPT;
+          c0[i] = rmul(e0, herm_load<T, NX>(fv, kr, y0, ny, a.kin, active && kr <= NX / 2));
+          c1[i] = rmul(e1, herm_load<T, NX>(fv, kr, y0 + 1, ny, a.kin, active && kr <= NX / 2));
+        }
+      }
       const MirrorSlots<NX, TPT, XPad<T>::G> ms(t);
 #pragma unroll
       for (int q = 0; q < P; ++q) L[ms.k(q)] = w[0][q];
@@ -488,8 +507,14 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
           const int kr = t + i * TPT;
           if (kr < a.kout) {
             const cplx<T> Wk = L[ms.k(i)], Wm = L[ms.m(i)];
-            at(o, boff32(kr, y0, ny)) = split_row(Wk, Wm, 0);
-            at(o, boff32(kr, y0 + 1, ny)) = split_row(Wk, Wm, 1);
+            cplx<T> r0 = split_row(Wk, Wm, 0), r1 = split_row(Wk, Wm, 1);
+            if (JET && gradient) {
+              const T kv = krwave(g, kr);
+              r0 = mk(kv * r0.im - c0[i].re, -kv * r0.re - c0[i].im);
+              r1 = mk(kv * r1.im - c1[i].re, -kv * r1.re - c1[i].im);
+            }
+            at(o, boff32(kr, y0, ny)) = r0;
+            at(o, boff32(kr, y0 + 1, ny)) = r1;
           }
         }
       }
@@ -512,20 +537,23 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
     }
     // with hsplit 1 where a thread group per field does not fit (K2P), workgroup row 0 forms u q and
     // row 1 v q (each transforms q itself)
-    const int half = a.hsplit == 1 ? (int)blockIdx.y : 2;
-    if (half != 1) {
+    const int half = NL == 1 && a.hsplit == 1 ? (int)blockIdx.y : 2;
+    auto product = [&](const cplx<T>* f, cplx<T>* o, T U0, T U1, bool gradient) {
       cplx<T> w[1][P];
-      inverse_rows(fu, w);
+      inverse_rows(f, w);
 #pragma unroll
-      for (int q = 0; q < P; ++q) w[0][q] = mk(w[0][q].re * q0[q], -w[0][q].im * q1[q]);   // u q, both rows
-      forward_rows(a.out, w);
-    }
-    if (half != 0) {
-      cplx<T> w[1][P];
-      inverse_rows(fv, w);
-#pragma unroll
-      for (int q = 0; q < P; ++q) w[0][q] = mk(w[0][q].re * q0[q], -w[0][q].im * q1[q]);   // v q, both rows
-      forward_rows(a.out + a.ostride, w);
+      for (int q = 0; q < P; ++q)
+        w[0][q] = JET ? mk((w[0][q].re + U0) * q0[q], (U1 - w[0][q].im) * q1[q])
+                      : mk(w[0][q].re * q0[q], -w[0][q].im * q1[q]);
+      forward_rows(o, w, gradient);
+    };
+    if constexpr (JET) {                               // v first: u's spectrum needs v's lines once more
+      const bool bg = active;
+      if (half != 0) product(fv, out + a.ostride, (T)0, (T)0, false);
+      if (half != 1) product(fu, out, bg ? a.Uy[jl * ny + y0] : (T)0, bg ? a.Uy[jl * ny + y0 + 1] : (T)0, true);
+    } else {
+      if (half != 1) product(fu, out, (T)0, (T)0, false);                  // u q, both rows
+      if (half != 0) product(fv, out + a.ostride, (T)0, (T)0, false);      // v q, both rows
     }
   } else {
     // ---- advection with background gradients: per layer, u, v, q -> (u q, v q, u Qx + v Qy) ----
@@ -665,8 +693,8 @@ __device__ __forceinline__ void k2_body(const K2Args<T>& a, int blk, cplx<T>* __
 // K2 for rows whose length nx is not a power of two (even, 18..GEN_MAX): the fields, products,
 // packing and outputs of k2_body's modes with the runtime nx in the kernel of NX = pow2_ceil(nx),
 // dft_even in place of the Stockham transform.  Always two rows of one field per transform;
-// a layer (K2_ADVECT_FULL), a product (K2_ADVECT) or a field (forward-in, inverse-out) has its own
-// workgroup row, which these small grids need to fill the GPU.
+// a layer (K2_ADVECT_FULL), a product (K2_ADVECT, K2_ADVECT_Y) or a field (forward-in, inverse-out) has its
+// own workgroup row, which these small grids need to fill the GPU.
 // ---------------------------------------------------------------------------
 template <int NX> struct K2G {
   static constexpr int P = 4, TPT = NX / P, G = TPT >= 64 ? 1 : 64 / TPT;
@@ -756,11 +784,13 @@ void k2_gen_kernel(const K2Args<T> a) {
     store(a.out + f * a.ostride, r0, r1);
   } else {
     // K2_ADVECT: u (q [+ eta]) in workgroup row 0, v (q [+ eta]) in row 1 (src/twodnavierstokes.jl:262-270,
-    // src/singlelayerqg.jl:368-375); K2_ADVECT_FULL, one layer per workgroup row: u += U,
+    // src/singlelayerqg.jl:368-375); K2_ADVECT_Y: two such rows per layer, u += U and -i kr (u q)^ - Qy v^
+    // in the first; K2_ADVECT_FULL, one layer per workgroup row: u += U,
     // (-i kr (u q)^ - (u Qx + v Qy)^, (v q)^) (src/multilayerqg.jl:695-731), or with `linear` U q in place of
     // u q and no v q (src/multilayerqg.jl:744-779)
     constexpr bool FULL = MODE == K2_ADVECT_FULL;
-    const int jl = FULL ? (int)blockIdx.y : 0, half = FULL ? 0 : (int)blockIdx.y;
+    constexpr bool JET = MODE == K2_ADVECT_Y;
+    const int jl = FULL ? (int)blockIdx.y : (JET ? (int)blockIdx.y >> 1 : 0), half = FULL ? 0 : (int)blockIdx.y & 1;
     const cplx<T>* in = a.in + (long)(3 * jl) * a.fstride;
     cplx<T>* out = a.out + (long)(2 * jl) * a.ostride;
     T q0[P], q1[P];
@@ -770,7 +800,7 @@ void k2_gen_kernel(const K2Args<T> a) {
       q0[q] = w[0][q].re;
       q1[q] = -w[0][q].im;
       const int x = t + TPT * q;
-      if (!FULL && a.eta != nullptr && x < nx) {
+      if (MODE == K2_ADVECT && a.eta != nullptr && x < nx) {
         q0[q] = q0[q] + a.eta[(long)y0 * nx + x];
         q1[q] = q1[q] + a.eta[(long)(y0 + 1) * nx + x];
       }
@@ -778,8 +808,26 @@ void k2_gen_kernel(const K2Args<T> a) {
     inverse_rows(in + (half ? a.fstride : 0), w);
     if constexpr (!FULL) {
 #pragma unroll
-      for (int q = 0; q < P; ++q) w[0][q] = mk(w[0][q].re * q0[q], -w[0][q].im * q1[q]);
+      for (int q = 0; q < P; ++q) {
+        const T U0 = JET && !half ? a.Uy[jl * ny + y0] : (T)0, U1 = JET && !half ? a.Uy[jl * ny + y0 + 1] : (T)0;
+        w[0][q] = JET ? mk((w[0][q].re + U0) * q0[q], (U1 - w[0][q].im) * q1[q])
+                      : mk(w[0][q].re * q0[q], -w[0][q].im * q1[q]);
+      }
       forward_split(w, r0, r1);
+      if (JET && !half) {
+        const cplx<T>* fv = in + a.fstride;
+        const T e0 = (T)nx * a.Qy1[jl * ny + y0], e1 = (T)nx * a.Qy1[jl * ny + y0 + 1];
+#pragma unroll
+        for (int i = 0; i < MAXI; ++i) {
+          const int kr = t + i * TPT;
+          if (kr >= a.kout) continue;
+          cplx<T> c0 = kr < a.kin ? at(fv, boff32(kr, y0, ny)) : czero<T>(), c1 = kr < a.kin ? at(fv, boff32(kr, y0 + 1, ny)) : czero<T>();
+          if (kr == 0 || 2 * kr == nx) { c0.im = 0; c1.im = 0; }
+          const T kv = krwave(g, kr);
+          r0[i] = mk(kv * r0[i].im - c0.re * e0, -kv * r0[i].re - c0.im * e0);
+          r1[i] = mk(kv * r1[i].im - c1.re * e1, -kv * r1[i].re - c1.im * e1);
+        }
+      }
       store(out + (half ? a.ostride : 0), r0, r1);
     } else {
       T u0[P], u1[P];
@@ -826,12 +874,13 @@ void k2_gen_kernel(const K2Args<T> a) {
 template <typename T, int NX>
 void k2_gen(const K2Args<T>& a, hipStream_t s) {
   constexpr int G = K2G<NX>::G;
-  const int rows = a.mode == K2_ADVECT ? 2 : (a.mode == K2_ADVECT_FULL ? a.g.nlayers : a.nfields);
+  const int rows = a.mode == K2_ADVECT ? 2 : a.mode == K2_ADVECT_Y ? 2 * a.g.nlayers : (a.mode == K2_ADVECT_FULL ? a.g.nlayers : a.nfields);
   if (rows <= 0) return;
   const dim3 grid((a.g.ny / 2 + G - 1) / G, rows), blk(G * K2G<NX>::TPT);
   switch (a.mode) {
     case K2_ADVECT: GF_LAUNCH((k2_gen_kernel<T, NX, K2_ADVECT>), grid, blk, 0, s, a); break;
     case K2_ADVECT_FULL: GF_LAUNCH((k2_gen_kernel<T, NX, K2_ADVECT_FULL>), grid, blk, 0, s, a); break;
+    case K2_ADVECT_Y: GF_LAUNCH((k2_gen_kernel<T, NX, K2_ADVECT_Y>), grid, blk, 0, s, a); break;
     case K2_INVERSE_OUT: GF_LAUNCH((k2_gen_kernel<T, NX, K2_INVERSE_OUT>), grid, blk, 0, s, a); break;
     case K2_FORWARD_IN: GF_LAUNCH((k2_gen_kernel<T, NX, K2_FORWARD_IN>), grid, blk, 0, s, a); break;
     default: break;
@@ -843,7 +892,7 @@ void k2_gen(const K2Args<T>& a, hipStream_t s) {
 #endif
 template <typename T, int NX, int P, int G, int MODE, int NL>
 __global__ __launch_bounds__(G * (NX / P))
-__attribute__((amdgpu_waves_per_eu(MODE == K2_ADVECT ? GF_K2_ADVECT_WAVES : GF_K2_WAVES)))
+__attribute__((amdgpu_waves_per_eu(MODE == K2_ADVECT || MODE == K2_ADVECT_Y ? GF_K2_ADVECT_WAVES : GF_K2_WAVES)))
 void k2_kernel(const K2Args<T> a) {
   __shared__ cplx<T> lds[G * LdsN<NX>::value];
   __shared__ cplx<T> tw[TwPlan<NX, P>::size()];
@@ -861,10 +910,12 @@ void k2_kernel(const K2Args<T> a) {
 // side by side too, so the chain is two transforms deep instead of five (or three where the
 // products had a workgroup each, every one transforming q again).  With P chosen so that a group
 // is one wave, its exchanges need no barrier (X_WAVE).  The layers of a multi-layer problem are
-// workgroup rows.  FULL: advection with background gradients (k2_body's K2_ADVECT_FULL).
+// workgroup rows.  K2_ADVECT_FULL: the third product u Qx + v Qy in group 2; K2_ADVECT_Y: group 0 subtracts
+// Qy v^ from its spectrum, group 2 is done when q is.
 // FP64 per launch, against the two workgroup rows of three transforms before: 64^2 5.2 -> 4.4 us, 128^2
 // 5.8 -> 4.6, 256^2 6.5 -> 4.7, 512^2 8.5 -> 7.0; MultiLayerQG 512^2 x 3, against a layer per workgroup row,
-// 17.4 -> 16.4.
+// 17.4 -> 16.4 and without topography (K2_ADVECT_Y) 13.2; U(y) at 1024^2, K2_ADVECT_FULL and K2_ADVECT_Y, 29.4
+// and 19.1.
 template <int NX, int P> struct K2P {
   static constexpr int TPT = NX / P;
   static constexpr int G = TPT >= 64 ? 1 : 64 / TPT;   // row pairs per group: whole waves
@@ -872,9 +923,10 @@ template <int NX, int P> struct K2P {
   static constexpr int X = GT == 64 ? X_WAVE : X_LDS;
   static constexpr bool fits(int size) { return 3 * GT <= 1024 && 3 * G * LdsN<NX>::value * size <= 120 * 1024; }
 };
-template <typename T, int NX, int P, bool FULL>
+template <typename T, int NX, int P, int MODE>
 __device__ __forceinline__ void k2_group_body(const K2Args<T>& a, int blk, int jl, cplx<T>* __restrict__ lds, cplx<T>* __restrict__ tw) {
   using K = K2P<NX, P>;
+  constexpr bool FULL = MODE == K2_ADVECT_FULL, JET = MODE == K2_ADVECT_Y;
   constexpr int TPT = K::TPT, G = K::G, X = K::X, PG = XPad<T>::G;
   constexpr int MAXI = (NX / 2 + 1 + TPT - 1) / TPT;
   constexpr int QH = P / 2 + 1;                        // the q with TPT q <= NX/2
@@ -918,7 +970,7 @@ __device__ __forceinline__ void k2_group_body(const K2Args<T>& a, int blk, int j
   fft_forward<T, NX, P, 1, false, X>(w, L, t, tw);     // row y0 = Re, row y0 + 1 = -Im
 #pragma unroll
   for (int q = 0; q < P; ++q) w[0][q] = conj(w[0][q]);  // (row y0, row y0 + 1)
-  if (!FULL && grp == 2 && a.eta != nullptr && active) {
+  if (MODE == K2_ADVECT && grp == 2 && a.eta != nullptr && active) {
 #pragma unroll
     for (int q = 0; q < P; ++q) {
       const int x = t + TPT * q;
@@ -933,10 +985,12 @@ __device__ __forceinline__ void k2_group_body(const K2Args<T>& a, int blk, int j
   if constexpr (!FULL) {
     if (grp == 2 && X == X_WAVE) return;               // (waves that share barriers stay)
     const cplx<T>* Q = buffer(2) + padg<PG>(t);
+    T U0 = 0, U1 = 0;
+    if (JET && grp == 0 && active) { U0 = a.Uy[jl * ny + y0]; U1 = a.Uy[jl * ny + y0 + 1]; }
 #pragma unroll
     for (int q = 0; q < P; ++q) {
       const cplx<T> qv = Q[padg<PG>(TPT * q)];
-      w[0][q] = mk(w[0][q].re * qv.re, w[0][q].im * qv.im);
+      w[0][q] = JET ? mk((w[0][q].re + U0) * qv.re, (w[0][q].im + U1) * qv.im) : mk(w[0][q].re * qv.re, w[0][q].im * qv.im);
     }
     if constexpr (X != X_WAVE) lds_barrier();          // group 2's buffer is read: it may transform along
   } else {
@@ -972,6 +1026,17 @@ __device__ __forceinline__ void k2_group_body(const K2Args<T>& a, int blk, int j
     }
     lds_barrier();                                     // the rows are read: the buffers are free
   }
+  cplx<T> c0[JET ? MAXI : 1], c1[JET ? MAXI : 1];      // (v Qy)^ = Qy v^, from the spectrum K1 left
+  if (JET && grp == 0) {
+    const cplx<T>* fv = a.in + (long)(3 * jl + 1) * a.fstride;
+    const T e0 = active ? (T)NX * a.Qy1[jl * ny + y0] : (T)0, e1 = active ? (T)NX * a.Qy1[jl * ny + y0 + 1] : (T)0;
+#pragma unroll
+    for (int i = 0; i < (JET ? MAXI : 1); ++i) {
+      const int kr = t + i * TPT;
+      c0[i] = rmul(e0, herm_load<T, NX>(fv, kr, y0, ny, a.kin, active && kr <= NX / 2));
+      c1[i] = rmul(e1, herm_load<T, NX>(fv, kr, y0 + 1, ny, a.kin, active && kr <= NX / 2));
+    }
+  }
   fft_forward<T, NX, P, 1, false, X>(w, L, t, tw);     // of (row y0 + i row y0 + 1)
   const MirrorSlots<NX, TPT, PG> ms(t);
 #pragma unroll
@@ -985,6 +1050,14 @@ __device__ __forceinline__ void k2_group_body(const K2Args<T>& a, int blk, int j
       const cplx<T> Wk = L[ms.k(i)], Wm = L[ms.m(i)];
       r0[i] = split_row(Wk, Wm, 0);
       r1[i] = split_row(Wk, Wm, 1);
+    }
+  }
+  if (JET && grp == 0) {
+#pragma unroll
+    for (int i = 0; i < (JET ? MAXI : 1); ++i) {
+      const T kv = krwave(g, t + i * TPT);
+      r0[i] = mk(kv * r0[i].im - c0[i].re, -kv * r0[i].re - c0[i].im);
+      r1[i] = mk(kv * r1[i].im - c1[i].re, -kv * r1[i].re - c1[i].im);
     }
   }
   if constexpr (FULL) {
@@ -1024,12 +1097,12 @@ __device__ __forceinline__ void k2_group_body(const K2Args<T>& a, int blk, int j
   }
 }
 
-template <typename T, int NX, int P, bool FULL>
+template <typename T, int NX, int P, int MODE>
 __global__ __launch_bounds__((3 * K2P<NX, P>::GT)) __attribute__((amdgpu_waves_per_eu(2)))
 void k2_group_kernel(const K2Args<T> a) {
   __shared__ cplx<T> lds[3 * K2P<NX, P>::G * LdsN<NX>::value];
   __shared__ cplx<T> tw[TwPlan<NX, P>::size()];
-  k2_group_body<T, NX, P, FULL>(a, xcd_block(blockIdx.x, gridDim.x), (int)blockIdx.y, lds, tw);
+  k2_group_body<T, NX, P, MODE>(a, xcd_block(blockIdx.x, gridDim.x), (int)blockIdx.y, lds, tw);
 }
 
 // ---------------------------------------------------------------------------
@@ -1654,7 +1727,7 @@ void k1_n(const K1Args<T>& a, hipStream_t s) {
 template <typename T, int N, int NL, int P>
 void k2_np(const K2Args<T>& a, hipStream_t s) {
   constexpr int G = GW<N, P>::G;
-  const int gy = (NL > 1 && a.lsplit) ? NL : ((NL == 1 && a.hsplit == 1 && a.mode == K2_ADVECT) ? 2 : 1);
+  const int gy = (NL > 1 && a.lsplit) ? NL : ((NL == 1 && a.hsplit == 1 && (a.mode == K2_ADVECT || a.mode == K2_ADVECT_Y)) ? 2 : 1);
   const dim3 grid((a.g.ny / 2 + G - 1) / G, gy), blk(G * (N / P));
   if constexpr (NL == 1 && BW == 2 && N / P >= 64) {   // whole waves: the staging is issued per wave
     if (a.mode == K2_ADVECT && a.hsplit == 2) {   // the staged x pass (a schedule option)
@@ -1665,11 +1738,12 @@ void k2_np(const K2Args<T>& a, hipStream_t s) {
   if constexpr (K2P<N, P>::fits(sizeof(cplx<T>))) {
     // a thread group per field: the split the schedule asks for, and every multi-layer problem
     // (a layer per workgroup row) up to 1024 points
-    const bool full = a.mode == K2_ADVECT_FULL;
-    if (NL > 1 ? (full && a.lsplit && N <= 1024) : (a.hsplit == 1 && (full || a.mode == K2_ADVECT))) {
+    const bool bg = a.mode == K2_ADVECT_FULL || a.mode == K2_ADVECT_Y;
+    if (NL > 1 ? (bg && a.lsplit && N <= 1024) : (a.hsplit == 1 && (bg || a.mode == K2_ADVECT))) {
       const dim3 gg((a.g.ny / 2 + K2P<N, P>::G - 1) / K2P<N, P>::G, NL), bb(3 * K2P<N, P>::GT);
-      if (full) GF_LAUNCH((k2_group_kernel<T, N, P, true>), gg, bb, 0, s, a);
-      else if constexpr (NL == 1) GF_LAUNCH((k2_group_kernel<T, N, P, false>), gg, bb, 0, s, a);
+      if (a.mode == K2_ADVECT_FULL) GF_LAUNCH((k2_group_kernel<T, N, P, K2_ADVECT_FULL>), gg, bb, 0, s, a);
+      else if (a.mode == K2_ADVECT_Y) GF_LAUNCH((k2_group_kernel<T, N, P, K2_ADVECT_Y>), gg, bb, 0, s, a);
+      else if constexpr (NL == 1) GF_LAUNCH((k2_group_kernel<T, N, P, K2_ADVECT>), gg, bb, 0, s, a);
       return;
     }
   }
@@ -1677,11 +1751,13 @@ void k2_np(const K2Args<T>& a, hipStream_t s) {
     return;                               // (multi-layer problems always have a layer per workgroup row)
   } else if constexpr (P != PY<N>::P) {          // a tuned schedule: the calcN modes only
     if (a.mode == K2_ADVECT) { if constexpr (NL == 1) GF_LAUNCH((k2_kernel<T, N, P, G, K2_ADVECT, 1>), grid, blk, 0, s, a); }
-    else GF_LAUNCH((k2_kernel<T, N, P, G, K2_ADVECT_FULL, NL>), grid, blk, 0, s, a);
+    else if (a.mode == K2_ADVECT_Y) GF_LAUNCH((k2_kernel<T, N, P, G, K2_ADVECT_Y, NL>), grid, blk, 0, s, a);
+    else if constexpr (P < 16) GF_LAUNCH((k2_kernel<T, N, P, G, K2_ADVECT_FULL, NL>), grid, blk, 0, s, a);
   } else {
     switch (a.mode) {
       case K2_ADVECT: if constexpr (NL == 1) GF_LAUNCH((k2_kernel<T, N, P, G, K2_ADVECT, 1>), grid, blk, 0, s, a); break;
       case K2_ADVECT_FULL: GF_LAUNCH((k2_kernel<T, N, P, G, K2_ADVECT_FULL, NL>), grid, blk, 0, s, a); break;
+      case K2_ADVECT_Y: GF_LAUNCH((k2_kernel<T, N, P, G, K2_ADVECT_Y, NL>), grid, blk, 0, s, a); break;
       case K2_INVERSE_OUT: if constexpr (NL == 1) GF_LAUNCH((k2_kernel<T, N, P, G, K2_INVERSE_OUT, 1>), grid, blk, 0, s, a); break;
       case K2_FORWARD_IN: if constexpr (NL == 1) GF_LAUNCH((k2_kernel<T, N, P, G, K2_FORWARD_IN, 1>), grid, blk, 0, s, a); break;
       default: break;
@@ -1693,19 +1769,20 @@ void k2_n(const K2Args<T>& a, hipStream_t s) {
   if constexpr (N <= GEN_MAX) {
     if (a.g.nx != N) { k2_gen<T, N>(a, s); return; }   // a row length below N
   }
-  const bool tuned = NL == 1 && (a.mode == K2_ADVECT || a.mode == K2_ADVECT_FULL) && a.p != 0 &&
+  const bool tuned = NL == 1 && (a.mode == K2_ADVECT || a.mode == K2_ADVECT_FULL || a.mode == K2_ADVECT_Y) && a.p != 0 &&
                      a.p != PY<N>::P && PCand<N>::has(a.p);
   if constexpr (NL == 1) {
     if (tuned && a.p == 4) { if constexpr (PCand<N>::has(4) && PY<N>::P != 4) { k2_np<T, N, 1, 4>(a, s); return; } }
     if (tuned && a.p == 8) { if constexpr (PCand<N>::has(8) && PY<N>::P != 8) { k2_np<T, N, 1, 8>(a, s); return; } }
-    // (with background gradients a thread holds three products: 16 points of them spill, so those
-    // run at 8 where the schedule says 16)
-    if (tuned && a.p == 16 && a.mode == K2_ADVECT) { if constexpr (PCand<N>::has(16) && PY<N>::P != 16) { k2_np<T, N, 1, 16>(a, s); return; } }
+    // (with gradients that depend on x a thread holds three products: 16 points of them spill, so
+    // those run at 8 where the schedule says 16; so does FP32 with gradients in y, where 16 is no faster:
+    // 33.6 and 33.9 us at 2048^2, FP64 43.5 and 46.9)
+    if (tuned && a.p == 16 && (a.mode == K2_ADVECT || (a.mode == K2_ADVECT_Y && sizeof(T) == 8))) { if constexpr (PCand<N>::has(16) && PY<N>::P != 16) { k2_np<T, N, 1, 16>(a, s); return; } }
   }
   (void)tuned;
   if constexpr (NL > 1) {
     // multi-layer x pass: a group of one wave per field up to 512 points
-    if (a.mode == K2_ADVECT_FULL && N >= 64) { k2_np<T, N, NL, PMX<N>::P>(a, s); return; }
+    if ((a.mode == K2_ADVECT_FULL || a.mode == K2_ADVECT_Y) && N >= 64) { k2_np<T, N, NL, PMX<N>::P>(a, s); return; }
   }
   k2_np<T, N, NL, PY<N>::P>(a, s);
 }

@@ -163,3 +163,35 @@ def test_two_launch_adjoint_matches_the_separate_kernels(gf, n):
     (J0, g0, nu0), (J1, g1, nu1) = got
     assert abs(J0 - J1) <= 1e-13 * abs(J1) and abs(nu0 - nu1) <= 1e-11 * abs(nu1)
     assert rel(g0, g1) < 1e-12
+
+
+# gradients that depend on y only: the x pass multiplies v's spectrum by Qy; with a topography (here one
+# of height 1e-200) it transforms u Qx + v Qy.  Both round each of at most 2 log2(nx ny) butterfly levels and a handful of
+# products once; the sum of the three terms cancels to no less than a tenth of its largest one.
+@pytest.mark.parametrize("nl,nx,ny", [(1, 32, 32), (1, 64, 32), (1, 512, 64), (1, 1024, 32), (1, 2048, 32), (1, 4096, 16), (1, 34, 62),
+                                      (1, 126, 32), (1, 64, 30), (2, 32, 64), (3, 512, 32), (2, 1024, 32), (2, 2048, 32), (2, 18, 30),
+                                      (5, 128, 126), (8, 64, 32)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_gradients_in_y_only_match_transformed_ones(gf, nl, nx, ny, dtype):
+    eps = np.finfo(dtype).eps
+    tol = 10 * (2 * np.log2(nx * ny) + 10) * eps
+    y = 2 * np.pi * np.arange(ny) / ny
+    kw = dict(nx=nx, ny=ny, β=1.5, μ=0.05, T=dtype)
+    s = np.stack([state(ny, nx, dtype, seed=k) for k in range(nl)])
+    for aliased, U in ((1 / 3, 0.2), (0.0, 0.3)):
+        out = []
+        for eta in (np.full((ny, nx), 1e-200), None):
+            more = dict(kw, aliased_fraction=aliased)
+            if nl == 1:
+                p = gf.SingleLayerQG.Problem(gf.GPU(), U=U * np.cos(y), eta=eta, **more)
+            else:
+                prof = U * np.cos(y)[None, :] * np.arange(1, nl + 1)[:, None] / nl
+                p = gf.MultiLayerQG.Problem(nl, gf.GPU(), f0=1.0, U=prof, H=[1.0 / nl] * nl, b=list(-0.2 * np.arange(nl)),
+                                            eta=eta, **more)
+            splits = [(0, 0, 0), (0, 1, 0)] if nl == 1 and (nx & (nx - 1)) == 0 and (ny & (ny - 1)) == 0 else [None]
+            for sp in splits:
+                if sp is not None:
+                    gf.set_splits(p, *sp)
+                out.append(p.calcN(s if nl > 1 else s[0])[0])
+        for o in out[1:]:
+            assert rel(o, out[0]) < tol
