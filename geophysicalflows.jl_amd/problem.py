@@ -435,8 +435,8 @@ class Ensemble:
     ``(SingleLayerQG.Problem, dict(nx=64, β=10.0, stepper="FilteredRK4", dt=0.01))``;
     sizes may differ.  ``ens.problems[i]`` is an ordinary ``Problem`` bound to member
     ``i`` (``set_q``, ``updatevars``, ``sol`` and diagnostics work on it);
-    ``stepforward(ens, n)`` advances every member with one launch per kernel class
-    and stage, ``stepforward(ens.problems[i], n)`` advances member ``i`` alone.
+    ``stepforward(ens, n)`` advances every member with two launches per stage,
+    ``stepforward(ens.problems[i], n)`` advances member ``i`` alone.
     The reference has no such object: an ensemble there is a loop over Problems.
     """
 

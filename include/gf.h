@@ -170,15 +170,17 @@ int gf_set_schedule(gf_ctx* ctx, int p_k1, int p_k2, int p_k3);
 int gf_get_schedule(gf_ctx* ctx, int* p_k1, int* p_k2, int* p_k3);
 
 /* Workgroup splits for single-layer problems (0 off, 1 on), part of the schedule:
- *   k1_fields:  K1 gives each of u, v, q its own row of workgroups;
- *   k2_halves:  K2 forms u q and v q in two rows of workgroups, each transforming q itself (1),
+ *   k1_fields:  K1 gives each of u, v, q its own row of workgroups, and the fused pass that steps run in
+ *               place of K3 and the next K1 its own thread group;
+ *   k2_halves:  K2 gives each of u, v, q its own thread group, or where three groups do not fit forms
+ *               u q and v q in two rows of workgroups, each transforming q itself (1),
  *               or walks row pairs persistently, each field's rows loaded straight into LDS one
  *               field ahead of the transforms (2; TwoDNavierStokes and SingleLayerQG without a
  *               varying U, nx / P_K2 >= 64; the unsplit pass runs elsewhere);
  *   k3_columns: K3 gives each spectral column its own workgroup instead of a column pair, where
  *               a column's ny / P_K3 threads fill a 64-lane wave (ignored elsewhere).
- * Workgroups are regrouped only: the results are the same bit for bit, except that k2_halves = 2
- * may round FP64 products differently (agreement to about 1e-16 relative). */
+ * Workgroups are regrouped only: the results are the same bit for bit, except that k2_halves may
+ * round differently (agreement to a few roundings). */
 int gf_set_splits(gf_ctx* ctx, int k1_fields, int k2_halves, int k3_columns);
 int gf_get_splits(gf_ctx* ctx, int* k1_fields, int* k2_halves, int* k3_columns);
 
@@ -245,7 +247,7 @@ int gf_kernel_bytes(const gf_ctx* ctx, int k, int full, double* bytes);
  * FP32, for all; TwoDNS, SingleLayerQG or one-layer MultiLayerQG; square grids with
  * n in 32..512, sizes may differ; one stepper for all, AB3 included; any forcing
  * kind but the time-harmonic one).  gf_step on the ensemble advances every member
- * with one launch per kernel class and stage covering all of them.  With ring
+ * with two launches per stage covering all of them.  With ring
  * forcing or AB3 every member must be at the same step (GF_EINVAL otherwise): the
  * forcing's step number and the AB3 start-up are shared.
  * gf_ctx_instance returns a borrowed handle for member i, valid until the
